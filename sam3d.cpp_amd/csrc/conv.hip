@@ -65,6 +65,7 @@ struct XformArgs {
     int32_t children;  // output row r reads x row r >> 3 and adds slot_offset[r & 7]
     const float *slot_offset;
     const float *scale, *shift;
+    uint32_t *fold_state;  // folded runs: the tile count to clear, the flag for infinities and NaN
 };
 
 template <class T>
@@ -83,6 +84,7 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
     constexpr int E = 16 / sizeof(T);
     const uint32_t ppr = static_cast<uint32_t>(a.cin) / E;
     const uint32_t total = static_cast<uint32_t>(a.rows) * ppr;
+    if (sizeof(T) == 2 && a.fold_state && blockIdx.x == 0 && threadIdx.x == 0) a.fold_state[kFoldCount] = 0u;
     for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < total; u += gridDim.x * 256u) {
         const uint32_t r = u / ppr;
         const int32_t c0 = static_cast<int32_t>(u - r * ppr) * E;
@@ -132,6 +134,13 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
             for (int k = 0; k < 4; ++k)
                 w4[k] = static_cast<uint32_t>(f32_to_bf16(v[2 * k])) | (static_cast<uint32_t>(f32_to_bf16(v[2 * k + 1])) << 16);
             o = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+            if (a.fold_state) {
+                bool bad = false;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    bad = bad || (w4[k] & 0x7f80u) == 0x7f80u || (w4[k] & 0x7f800000u) == 0x7f800000u;
+                if (bad) a.fold_state[kFoldBadRows] = 1u;
+            }
         } else {
             o = make_uint4(__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
                            __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3]));
@@ -294,13 +303,21 @@ struct s3dx_conv {
     // that are part of a tile, grown on demand like xin.
     mutable void *sk_part = nullptr;
     mutable int64_t sk_part_bytes = 0;
+    // Folded runs (conv_fold.hip): the folded weights, their flag behind them,
+    // made in the first such run after set_weights; the state words and the
+    // parent map's records, made in every run.  Like xin, which every such
+    // layer has.
+    mutable void *w_fold = nullptr;
+    mutable bool w_fold_ready = false;
+    mutable void *fold = nullptr;
+    mutable int64_t fold_bytes = 0;
 
     bool transforms() const { return slot_offset != nullptr || pre_scale != nullptr; }
 
     ~s3dx_conv() {
         for (void *p : {w, w_split, static_cast<void *>(bias), static_cast<void *>(slot_offset),
                         static_cast<void *>(ln_w), static_cast<void *>(ln_b),
-                        static_cast<void *>(mod_scale), static_cast<void *>(mod_shift), xin, pre_ln, sk_part})
+                        static_cast<void *>(mod_scale), static_cast<void *>(mod_shift), xin, pre_ln, sk_part, w_fold, fold})
             if (p) (void)hipFree(p);
     }
 };
@@ -760,6 +777,25 @@ int gather_plan_rows(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
     return tiles <= device_cus() || stream_k_runs(conv->cin, n_out, p.grid.y) ? 128 : 64;
 }
 
+// Column blocks per workgroup of a run of folded parent rows, 0 for the
+// general kernel: a BF16 layer that reads repeated parent rows through an
+// affine + SiLU pass (so it has buffers of its own, see s3dx_conv_run),
+// writes BF16 rows (whose rounding hides the folding's) of all 8 children of
+// every parent with no LayerNorm or residual, and would run the 64-row halo
+// kernel.  What the map holds is checked on the device.
+int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_in, int64_t n_out,
+                   bool residual, bool y_bf16) {
+    if (!p.mfma || p.linear || !p.tl || p.tl->id != 21 || p.half_chunk || p.xf || conv->dtype != S3DX_BF16 ||
+        src.shift != 3 || !conv->pre_scale || conv->ln || residual || !y_bf16 || n_out != 8 * n_in ||
+        conv->cout % 32 != 0 || !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING"))
+        return 0;
+    const int blocks = conv->cout_pad / 32;
+    if (fold_weight_bytes(conv->cin, blocks) >= (int64_t(1) << 31) ||
+        (n_in + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31))
+        return 0;
+    return fold_blocks(conv->cin, blocks, p.nb, n_in, device_cus());
+}
+
 float *upload_f32(const float *host, size_t count) {
     if (!host) return nullptr;
     void *d = nullptr;
@@ -909,6 +945,7 @@ S3DX_API s3dx_status s3dx_conv_set_weights(s3dx_conv *conv, const float *host_we
         }
         if (conv->w) (void)hipFree(conv->w);
         conv->w = d;
+        conv->w_fold_ready = false;
         if (conv->w_split) (void)hipFree(conv->w_split);
         conv->w_split = nullptr;
         const int nbtot = conv->cout_pad / 32;
@@ -1121,8 +1158,38 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         const bool bf16_rows = conv->in_dtype != conv->dtype;  // BF16 rows into an FP32 layer
         require(!(bf16_rows && src.pre), "BF16 input rows do not combine with input transforms");
         const int64_t x_bytes = src.rows * conv->cin * static_cast<int64_t>(dtype_size(conv->in_dtype));
+        // The MFMA kernel reads the map and writes rows with 16-byte accesses.
+        const bool aligned16 = aligned(kmap, 16) && aligned(y, 16) && aligned(residual, 16);
+        // 16-byte pieces with 32-bit piece indices; else one element per thread.
+        const bool xvec = conv->cin % (bf ? 8 : 4) == 0 &&
+                          src.rows * (conv->cin / (bf ? 8 : 4)) < (int64_t(1) << 32) &&
+                          aligned(conv->pre_scale, 16) && aligned(conv->pre_shift, 16);
+        LaunchPlan plan = plan_launch(conv, x_bytes, n_out, aligned16, bf16_rows,
+                                      residual == nullptr && y_dtype == S3DX_BF16);
+        int fold = xvec ? fold_blocks_of(conv, plan, src, n_in, n_out, residual != nullptr, y_dtype == S3DX_BF16) : 0;
+        uint32_t *fold_state = nullptr, *fold_bad = nullptr;
+        void *fold_records = nullptr;
+        if (fold) {
+            const int64_t tiles = (n_in + 127) / 128;
+            const int64_t words = static_cast<int64_t>(round_up((kFoldList + tiles) * 4, 1024));
+            const int64_t fw = fold_weight_bytes(conv->cin, conv->cout_pad / 32);
+            const int64_t had = conv->fold_bytes;
+            try {
+                fold_state = static_cast<uint32_t *>(
+                    layer_buffer(conv->fold, conv->fold_bytes, words + tiles * kGatherPlanRecord128, s));
+                if (!conv->w_fold) hip_check(hipMalloc(&conv->w_fold, static_cast<size_t>(fw) + 16), "hipMalloc");
+                fold_records = reinterpret_cast<char *>(fold_state) + words;
+                fold_bad = reinterpret_cast<uint32_t *>(static_cast<char *>(conv->w_fold) + fw);
+                if (conv->fold_bytes != had) fill_u32(fold_state, kFoldList, 0u, s);
+            } catch (const oom_error &) {  // no room for the folding's buffers: the general kernel
+                (void)hipGetLastError();
+                fold_state = nullptr;
+                fold = 0;
+            }
+        }
         if (src.pre) {
             XformArgs xa{};
+            xa.fold_state = fold_state;
             xa.x = x;
             xa.out = transform_buffer(conv, x_bytes, s);
             xa.rows = src.rows;
@@ -1131,10 +1198,7 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             xa.slot_offset = conv->slot_offset;
             xa.scale = conv->pre_scale;
             xa.shift = conv->pre_shift;
-            // 16-byte pieces with 32-bit piece indices; else one element per thread.
-            const bool vec = conv->cin % (bf ? 8 : 4) == 0 &&
-                             src.rows * (conv->cin / (bf ? 8 : 4)) < (int64_t(1) << 32) &&
-                             aligned(conv->pre_scale, 16) && aligned(conv->pre_shift, 16);
+            const bool vec = xvec;
             const int64_t items = src.rows * (vec ? conv->cin / (bf ? 8 : 4) : conv->cin);
             const dim3 grid(static_cast<unsigned>(std::min<int64_t>((items + 255) / 256, 16384)));
             if (vec) {
@@ -1170,10 +1234,6 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         a.ln_b = conv->ln_b;
         a.mod_scale = conv->dmod_scale ? conv->dmod_scale : conv->mod_scale;
         a.mod_shift = conv->dmod_scale ? conv->dmod_shift : conv->mod_shift;
-        // The MFMA kernel reads the map and writes rows with 16-byte accesses.
-        const bool aligned16 = aligned(kmap, 16) && aligned(y, 16) && aligned(residual, 16);
-        LaunchPlan plan = plan_launch(conv, a.x_bytes, n_out, aligned16, bf16_rows,
-                                      residual == nullptr && y_dtype == S3DX_BF16);
         if (bf16_rows && !plan.linear) {
             // Other kernels read the layer's dtype: the rows are widened
             // (exactly) once, into the layer's buffer.
@@ -1193,6 +1253,25 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             if (plan.fn == pick_halo_bf16_planned(64) || plan.fn == pick_halo_bf16_planned(128) ||
                 plan.fn == pick_halo_bf16_planned(64, 3) || plan.stream_k)
                 a.plan = gplan->d;
+        }
+        if (fold) {
+            if (!conv->w_fold_ready) {
+                fill_u32(fold_bad, 1, 0u, s);
+                launch_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad / 32, fold_bad, s);
+                launch_check("fold_weights");
+                conv->w_fold_ready = true;
+            }
+            launch_fold_plan(kmap, n_in, fold_records, fold_state, fold_bad, s);
+            launch_check("fold_plan");
+            ConvArgs fa = a;
+            fa.w = conv->w_fold;
+            fa.plan = fold_records;
+            launch_conv_fold(fa, fold, s);
+            launch_check("conv_fold");
+            a.plan = nullptr;
+            launch_halo_listed(a, plan.nb, fold_state, s);
+            launch_check("conv_halo_listed");
+            return;
         }
         // A LayerNorm the epilogue cannot fuse runs as its own pass over the
         // conv's FP32 output (the layer's buffer), then modulate, SiLU and

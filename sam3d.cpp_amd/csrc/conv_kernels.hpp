@@ -107,6 +107,22 @@ void launch_kmap_plan(int rows, const int32_t *coords, int64_t n, int32_t missin
                       uint64_t workspace_bytes, void *plan, hipStream_t stream);
 constexpr int kGatherPlanRecord = 7168;      // 64-row tiles
 constexpr int kGatherPlanRecord128 = 18432;  // 128-row tiles
+// Folded convs over repeated parent rows (conv_fold.hip).  `state`: the words
+// below, then the list (one word per 128 parents); the count is cleared before
+// each run's plan, the flag by the listed pass that ends a run.
+constexpr int kFoldCount = 0;    // parent tiles left to the general kernel
+constexpr int kFoldBadRows = 1;  // a source row holds an infinity or NaN
+constexpr int kFoldList = 4;     // the tiles counted
+constexpr uint32_t kFoldGeneral = 2;  // record mode of those tiles
+int64_t fold_weight_bytes(int cin, int blocks);
+int fold_blocks(int cin, int blocks, int general_nb, int64_t n_parents, int64_t cus);
+// *bad: raised when a folded weight is no finite number.
+void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t *bad, hipStream_t stream);
+void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
+                      hipStream_t stream);
+void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
+// The general kernel (64-row tiles, nb column blocks) over the listed tiles.
+void launch_halo_listed(const ConvArgs &a, int nb, uint32_t *state, hipStream_t stream);
 // The FP32 1x1-layer kernel reading BF16 rows, else nullptr.
 KernelFn pick_linear_f32_bf16_rows(int nbt);
 // The same on BF16 MFMAs with three-term split weights (Cin = 16 * ksx,

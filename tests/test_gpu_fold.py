@@ -1,0 +1,124 @@
+"""Convs over repeated parent rows on the folded kernel (conv_fold.hip).
+
+A BF16 layer that gathers parent rows behind an affine + SiLU pass sums the
+weights of the offsets that reach one parent (two BF16 terms a sum) and
+multiplies 8 parents instead of 27 children.  Against the 27-offset kernel
+(S3DX_CONV_TILING=21): both accumulate in FP32 and round once to BF16, and the
+folded weights are within 2^-17 of the sums, so the outputs differ by at most
+one BF16 step here and there (rel-L2 far below 2^-9).  Parent tiles whose map
+is not a subdivide's, or rows that hold an infinity, go to the 27-offset
+kernel: those outputs are the same bits.
+"""
+import numpy as np
+import pytest
+
+from helpers import check_rel
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(s3dx, W, parents, cin, cout, silu=False, seed=70):
+    p = parents.shape[0]
+    _, kd = s3dx.subdivide2(s3dx.DeviceArray.from_host(parents), p, True)
+    x = W.round_bf16(W.normal_f32(seed, 1, (p, cin)))
+    scale, shift = W.normal_f32(seed, 2, (cin,), 0.2) + 1.0, W.normal_f32(seed, 3, (cin,), 0.2)
+    ds, dh = s3dx.DeviceArray.from_host(scale), s3dx.DeviceArray.from_host(shift)
+    w, b = W.conv_weight(seed, 4, cin, cout, layout="mesh"), W.normal_f32(seed, 5, (cout,), 0.1)
+    conv = (s3dx.SparseConv(cin, cout, 27, s3dx.BF16).set_weights(w, s3dx.WEIGHT_MESH, b).set_gather_parent(True)
+            .set_input_affine_silu(ds, dh).set_silu(silu))
+    return conv, kd.download(), x, w, b, scale, shift
+
+
+def _run(s3dx, W, conv, x, kmap, cout, n_out=None):
+    n = kmap.shape[0] if n_out is None else n_out
+    y = s3dx.DeviceArray((n, cout), np.uint16)
+    conv.run(s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(x)), x.shape[0], s3dx.DeviceArray.from_host(kmap), n, y,
+             s3dx.BF16)
+    return y.download()
+
+
+def _general(s3dx, W, monkeypatch, *args, **kw):
+    monkeypatch.setenv("S3DX_CONV_TILING", "21")
+    y = _run(s3dx, W, *args, **kw)
+    monkeypatch.delenv("S3DX_CONV_TILING")
+    return y
+
+
+@pytest.mark.parametrize("p,cin,cout,silu", [
+    (6007, 192, 96, False),   # one column block a workgroup; a ragged last parent tile
+    (20011, 192, 96, True),   # three
+    (12801, 64, 192, False),  # one chunk; a last tile of one parent
+    (9000, 128, 128, False),  # column blocks in twos
+    (4000, 768, 192, False),  # the mesh decoder's first level
+])
+def test_folded_matches_general_and_oracle(s3dx, O, W, monkeypatch, p, cin, cout, silu):
+    parents = W.shells_union(0)[:p]
+    conv, kmap, x, w, b, scale, shift = _setup(s3dx, W, parents, cin, cout, silu)
+    print(f"fold p={p} {cin}->{cout} silu={silu}", flush=True)
+    got = _run(s3dx, W, conv, x, kmap, cout)
+    assert np.array_equal(got, _run(s3dx, W, conv, x, kmap, cout)), "two runs differ"
+    want = _general(s3dx, W, monkeypatch, conv, x, kmap, cout)
+    g, v = W.bf16_bits_to_f32(got).reshape(got.shape), W.bf16_bits_to_f32(want).reshape(got.shape)
+    rel = float(np.linalg.norm(g - v) / np.linalg.norm(v))
+    print(f"  against the 27-offset kernel: rel-L2 {rel:.2e}, same bits {np.mean(got == want):.4f}", flush=True)
+    assert 0.0 < rel < 2.0 ** -11  # (0: the folded kernel did not run)
+    rows = np.sort(np.random.default_rng(1).choice(8 * p, 1500, replace=False))
+    rows = np.unique(np.concatenate([rows, [0, 1023, 1024, 8 * p - 1]]))
+    a = W.round_bf16(O.silu((x * scale + shift).astype(np.float32)))
+    km = np.where(kmap[rows] >= 0, kmap[rows] >> 3, -1).astype(np.int32)
+    ref = O.conv(a, km, p, W.round_bf16(w), 1, cout, b)
+    check_rel(g[rows], O.silu(ref) if silu else ref, 1e-2, "oracle")
+
+
+def test_maps_no_subdivide_made(s3dx, W, monkeypatch):
+    # Tiles with an entry that does not reach the parent its siblings reach
+    # run the 27-offset kernel (the same bits); the other tiles are folded.
+    p, cin, cout = 8000, 192, 96
+    conv, kmap, x, *_ = _setup(s3dx, W, W.shells_union(1)[:p], cin, cout)
+    bad = kmap.copy()
+    bad[8 * 130 + 3, 14] = -1            # tile 1: a neighbour taken away
+    bad[8 * 300 + 0, 26] = 8 * 4000 + 1  # tile 2: another parent's child
+    bad[8 * 4000:8 * 4128] = np.random.default_rng(2).integers(-1, 8 * p, (1024, 27), dtype=np.int32)  # tile 31 and 32
+    sib = bad.copy()
+    j = sib[8 * 700 + 5, 13]
+    sib[8 * 700 + 5, 13] = (j & ~7) | ((j + 3) & 7)  # a sibling: the same parent row, so still foldable
+    got, want = _run(s3dx, W, conv, x, bad, cout), _general(s3dx, W, monkeypatch, conv, x, bad, cout)
+    for t in (1, 2, 31, 32):
+        assert np.array_equal(got[1024 * t:1024 * (t + 1)], want[1024 * t:1024 * (t + 1)]), t
+    assert not np.array_equal(got[:1024], want[:1024])  # folded
+    assert np.array_equal(got, _run(s3dx, W, conv, x, sib, cout))
+    # every tile irregular, then the subdivide's map again
+    rnd = np.random.default_rng(3).integers(-1, 8 * p, kmap.shape, dtype=np.int32)
+    assert np.array_equal(_run(s3dx, W, conv, x, rnd, cout), _general(s3dx, W, monkeypatch, conv, x, rnd, cout))
+    none = np.full_like(kmap, -1)
+    assert np.array_equal(_run(s3dx, W, conv, x, none, cout), _general(s3dx, W, monkeypatch, conv, x, none, cout))
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout)[:1024], got[:1024])
+    # fewer rows than eight per parent: the general kernel
+    n = 8 * p - 8
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap[:n], cout, n), _general(s3dx, W, monkeypatch, conv, x, kmap[:n], cout, n))
+
+
+def test_infinities_new_weights_and_sizes(s3dx, W, monkeypatch):
+    # An infinite or NaN row sends the run to the 27-offset kernel (the folded
+    # sum's two terms may differ in sign); the next run folds again.  New
+    # weights are folded anew; a larger set, then the first again.
+    cin, cout = 192, 96
+    conv, kmap, x, w, b, *_ = _setup(s3dx, W, W.shells_union(2)[:7000], cin, cout)
+    first = _run(s3dx, W, conv, x, kmap, cout)
+    for v in (np.inf, -np.inf, np.nan):
+        xi = x.copy()
+        xi[500, 7] = v
+        assert np.array_equal(_run(s3dx, W, conv, xi, kmap, cout), _general(s3dx, W, monkeypatch, conv, xi, kmap, cout)), v
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), first)
+    conv.set_weights(2.0 * w, s3dx.WEIGHT_MESH, 2.0 * b)  # (twice: exact in BF16)
+    twice = _run(s3dx, W, conv, x, kmap, cout)
+    assert np.array_equal(W.bf16_bits_to_f32(twice), 2.0 * W.bf16_bits_to_f32(first))
+    big, kb, xb, *_ = _setup(s3dx, W, W.shells_union(2)[:12000], cin, cout)
+    conv.set_weights(w, s3dx.WEIGHT_MESH, b)
+    assert np.array_equal(_run(s3dx, W, conv, xb, kb, cout), _run(s3dx, W, big, xb, kb, cout))
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), first)
+    # a weight whose folded sum overflows: the 27-offset kernel
+    wh = w.copy()
+    wh[:, 0, 0] = 2.0e38
+    conv.set_weights(wh, s3dx.WEIGHT_MESH, b)
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), _general(s3dx, W, monkeypatch, conv, x, kmap, cout))
