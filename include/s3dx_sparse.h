@@ -242,8 +242,11 @@ S3DX_API s3dx_status s3dx_downsample_coords(const int32_t *coords, int64_t n, in
  * cannot span the row (Cout above 256, or not whole 32-column blocks) the
  * LayerNorm runs as a second pass over the conv's float32 output, kept in
  * another buffer the layer owns (n_out * Cout * 4 bytes, same rules).
- * Arithmetic: float32 inputs use FP32 MFMA/VALU; bfloat16 inputs use BF16 MFMA;
- * both accumulate in float32.  Deterministic (no atomics on outputs).
+ * Arithmetic: float32 inputs use FP32 MFMA/VALU, or, in 3x3x3 layers with
+ * records of the map at hand (a gather plan made for an FP32 layer, or input
+ * transforms, whose layers make their own), BF16 MFMA on three BF16 terms of
+ * every value, with no larger error against float64; bfloat16 inputs use BF16
+ * MFMA; all accumulate in float32.  Deterministic (no atomics on outputs).
  * ---------------------------------------------------------------------- */
 typedef struct s3dx_conv s3dx_conv;
 
@@ -329,8 +332,9 @@ S3DX_API s3dx_status s3dx_conv_run(const s3dx_conv *conv, const void *x, int64_t
  * in use.  create enqueues the build on `stream` and picks the records' tile
  * height from `conv`: 128 output rows when its halo kernel's 128-row tiles
  * fill the GPU's compute units in one pass (runs then use an 8-wave kernel
- * on those tiles; 18 KiB of device memory per 128 rows), else 64 rows (7
- * KiB per 64 rows); free releases it. */
+ * on those tiles; 18 KiB of device memory per 128 rows), or when it is an
+ * FP32 layer that runs as three BF16 terms, else 64 rows (7 KiB per 64
+ * rows); free releases it. */
 typedef struct s3dx_gather_plan s3dx_gather_plan;
 S3DX_API s3dx_status s3dx_gather_plan_create(const s3dx_conv *conv, int64_t n_in, const int32_t *kmap,
                                              int64_t n_out, s3dx_stream stream, s3dx_gather_plan **out,
@@ -363,7 +367,11 @@ S3DX_API s3dx_status s3dx_kmap_subm3_planned(const int32_t *coords, int64_t n, i
  * on 5,086 rows): with a 128-row plan those run in stream-K runs, equal runs
  * of (tile, 64-channel chunk) units one per CU, and a tile split between
  * runs adds its pieces in a fixed order, so results are deterministic but
- * rounded differently from the unplanned run (within BF16 rounding).
+ * rounded differently from the unplanned run (within BF16 rounding), and
+ * except for FP32 layers: with a 128-row plan last built for an FP32 layer
+ * they run as three BF16 terms where that is faster, deterministic and with no
+ * larger error against float64, but rounded differently (within 2e-6); with a
+ * plan built for a BF16 layer they ignore it.
  * Launches that do not use the halo kernel ignore the plan. */
 S3DX_API s3dx_status s3dx_conv_run_planned(const s3dx_conv *conv, const s3dx_gather_plan *plan, const void *x,
                                            int64_t n_in, const int32_t *kmap, int64_t n_out, const void *residual,

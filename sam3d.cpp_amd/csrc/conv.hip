@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
     constexpr int E = 16 / sizeof(T);
     const uint32_t ppr = static_cast<uint32_t>(a.cin) / E;
     const uint32_t total = static_cast<uint32_t>(a.rows) * ppr;
-    if (sizeof(T) == 2 && a.fold_state && blockIdx.x == 0 && threadIdx.x == 0) a.fold_state[kFoldCount] = 0u;
+    if (a.fold_state && blockIdx.x == 0 && threadIdx.x == 0) a.fold_state[kFoldCount] = 0u;
     for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < total; u += gridDim.x * 256u) {
         const uint32_t r = u / ppr;
         const int32_t c0 = static_cast<int32_t>(u - r * ppr) * E;
@@ -144,6 +144,11 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
         } else {
             o = make_uint4(__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
                            __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3]));
+            if (a.fold_state) {
+                // infinities, NaN, and what rounds to an infinite first term
+                auto none = [](uint32_t u) { return (u & 0x7fffffffu) >= 0x7f7f8000u; };
+                if (none(o.x) || none(o.y) || none(o.z) || none(o.w)) a.fold_state[kFoldBadRows] = 1u;
+            }
         }
         *reinterpret_cast<uint4 *>(static_cast<T *>(a.out) + static_cast<int64_t>(r) * a.cin + c0) = o;
     }
@@ -280,6 +285,9 @@ struct s3dx_conv {
     // FP32 1x1 layers: the weights again as three BF16 terms, for BF16 input
     // rows on BF16 MFMAs (linear_split_kernel); nullptr for other shapes.
     void *w_split = nullptr;
+    // FP32 3x3x3 layers: the weights as three BF16 terms (conv_f3.hip);
+    // nullptr for other layers, and when a weight has no finite terms.
+    void *w3 = nullptr;
     float *bias = nullptr;
     float *slot_offset = nullptr;
     bool gather_parent = false;
@@ -315,7 +323,7 @@ struct s3dx_conv {
     bool transforms() const { return slot_offset != nullptr || pre_scale != nullptr; }
 
     ~s3dx_conv() {
-        for (void *p : {w, w_split, static_cast<void *>(bias), static_cast<void *>(slot_offset),
+        for (void *p : {w, w_split, w3, static_cast<void *>(bias), static_cast<void *>(slot_offset),
                         static_cast<void *>(ln_w), static_cast<void *>(ln_b),
                         static_cast<void *>(mod_scale), static_cast<void *>(mod_shift), xin, pre_ln, sk_part, w_fold, fold})
             if (p) (void)hipFree(p);
@@ -328,6 +336,7 @@ struct s3dx_conv {
 struct s3dx_gather_plan {
     void *d = nullptr;
     int rows = 64;         // tile height of the records (64 or 128)
+    bool f32 = false;      // built for an FP32 layer: such layers then run as three BF16 terms
     int64_t capacity = 0;  // output rows the allocation covers
     int64_t n_out = 0, n_src = 0;
     int32_t shift = 0;
@@ -402,6 +411,7 @@ struct LaunchPlan {
     bool stream_k = false;    // the 8-wave kernel over equal runs of (group, tile, chunk) units
     int64_t sk_units = 0;     // (column group, tile, chunk) units of a stream-K launch
     int sk_groups = 0;        // its 128-column groups
+    int f3 = 0;               // FP32 as three BF16 terms: 32-column blocks per workgroup
     bool sk_splitk = false;   // the stream-K runs are the FP32 split-K kernel's (64-row tiles)
     unsigned smem = 0;      // dynamic LDS bytes
     unsigned threads = 256; // workgroup size
@@ -738,11 +748,60 @@ int stream_k_runs(int cin, int64_t n_out, int64_t groups) {
     return static_cast<int>(runs);
 }
 
+// Whether an FP32 layer can run as three BF16 terms: whole 32-channel chunks
+// and weights below 2 GiB in that form.
+bool f3_shape(const s3dx_conv *conv) {
+    return conv->dtype == S3DX_F32 && conv->in_dtype == S3DX_F32 && conv->kvol == kMaxKvol && conv->mfma &&
+           conv->cin % 32 == 0 && f3_weight_bytes(conv->cin, conv->cout_pad) < (int64_t(1) << 31);
+}
+
+// 32-column blocks per workgroup of that kernel for n_out rows, 0 where the
+// FP32 matrix instructions suit the size.  In microseconds: a pass of
+// workgroups (one per CU) takes 8 and, per 32-channel chunk, 5 per column block
+// and 1.7; the FP32 kernels about 95 TFLOP/s over all 27 offsets and 4.
+// Measured, three terms against FP32: 128 -> 128 on 2,000 rows 35 / 23 us,
+// 4,000 37 / 37, 8,000 45 / 72, 28,265 133 / 226; 64 -> 64 on 5,000 21 / 20,
+// 10,366 23 / 28; 1024 -> 1024 on 300 235 / 224, 5,086 1,441 / 2,004.
+int f3_blocks(const s3dx_conv *conv, int64_t n_out) {
+    const int blocks = conv->cout_pad / 32, chunks = conv->cin / 32;
+    const int64_t tiles = (n_out + 127) / 128, cus = device_cus();
+    double least = 4.0 + 54.0 * static_cast<double>(n_out) * conv->cin * conv->cout_pad / 95e6;
+    int best = 0;
+    for (int cg : {4, 2, 1}) {
+        if (blocks % cg != 0) continue;
+        const int64_t passes = (tiles * (blocks / cg) + cus - 1) / cus;
+        const double t = static_cast<double>(passes) * (8.0 + chunks * (5.0 * cg + 1.7));
+        if (t < least) {
+            best = cg;
+            least = t;
+        }
+        if (conv->ln && cg * 32 == conv->cout) break;  // the LayerNorm in the tile
+    }
+    return best;
+}
+
 // A planned launch: the halo kernel of the plan's tile height in place of
 // the unplanned halo kernel (64-row records: tiling 21 only; 128-row records:
 // tilings 20 and 21, on the 8-wave kernel, in stream-K runs where those pay).
 // Other launches are unchanged.
-void apply_gather_plan(LaunchPlan &p, const s3dx_gather_plan *g, int64_t n_out, bool bf16_rows, int cin) {
+void apply_gather_plan(LaunchPlan &p, const s3dx_conv *conv, const s3dx_gather_plan *g, int64_t n_out, bool bf16_rows) {
+    const int cin = conv->cin;
+    if (!bf16_rows && p.mfma && p.tl && !p.xf && g->f32 && g->rows == 128 && f3_shape(conv) &&
+        (conv->w3 || !conv->weights_set) && !std::getenv("S3DX_CONV_TILING")) {
+        const int cg = f3_blocks(conv, n_out);
+        if (cg) {
+            for (const Tiling &t : kTilings)
+                if (t.id == 25) p.tl = &t;
+            p.f3 = p.nb = cg;
+            p.kc = 32;
+            p.fn = pick_f3(cg);
+            p.threads = kHalo8Threads;
+            p.stream_k = p.sk_splitk = false;
+            p.fused_ln = conv->ln && cg * 32 == conv->cout;
+            p.grid = dim3(static_cast<unsigned>((n_out + 127) / 128), static_cast<unsigned>(conv->cout_pad / 32 / cg));
+            return;
+        }
+    }
     if (bf16_rows || !p.mfma || !p.tl || (p.tl->id != 20 && p.tl->id != 21)) return;
     if (g->rows == 64 && p.tl->id == 21) {
         p.fn = pick_halo_bf16_planned(64, p.nb);
@@ -763,6 +822,20 @@ void apply_gather_plan(LaunchPlan &p, const s3dx_gather_plan *g, int64_t n_out, 
     }
 }
 
+// An unplanned run of an FP32 layer that has buffers of its own (input
+// transforms): as three BF16 terms, with the map's 128-row records built in
+// the run where that pays (about 10 us).
+bool f3_own_plan(const s3dx_conv *conv, LaunchPlan &p, const Source &src, int64_t n_out) {
+    if (!src.pre || conv->dtype != S3DX_F32 || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
+        (n_out + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31) || n_out < 8192)
+        return false;
+    s3dx_gather_plan g;
+    g.rows = 128;
+    g.f32 = true;
+    apply_gather_plan(p, conv, &g, n_out, false);
+    return p.f3 != 0;
+}
+
 // Tile height of the gather plan for `conv`: 128-row records when the
 // layer runs a halo kernel and 128-row tiles fill the CUs in one pass (one
 // 8-wave workgroup per CU), else 64.  S3DX_PLAN_ROWS=64|128 forces it.
@@ -772,27 +845,37 @@ int gather_plan_rows(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
         if (r == 64 || r == 128) return r;
     }
     const LaunchPlan p = plan_launch(conv, x_bytes, n_out, true);
+    if (f3_shape(conv) && p.mfma && p.tl && !p.xf && !std::getenv("S3DX_CONV_TILING") && f3_blocks(conv, n_out)) return 128;
     if (!p.mfma || !p.tl || (p.tl->id != 20 && p.tl->id != 21) || p.nb != 4 || p.half_chunk) return 64;
     const int64_t tiles = (n_out + 127) / 128 * static_cast<int64_t>(p.grid.y);
     return tiles <= device_cus() || stream_k_runs(conv->cin, n_out, p.grid.y) ? 128 : 64;
 }
 
 // Column blocks per workgroup of a run of folded parent rows, 0 for the
-// general kernel: a BF16 layer that reads repeated parent rows through an
-// affine + SiLU pass (so it has buffers of its own, see s3dx_conv_run),
-// writes BF16 rows (whose rounding hides the folding's) of all 8 children of
-// every parent with no LayerNorm or residual, and would run the 64-row halo
-// kernel.  What the map holds is checked on the device.
+// general kernel: a layer that reads repeated parent rows through an affine +
+// SiLU pass (so it has buffers of its own, see s3dx_conv_run) and writes rows
+// of its own type of all 8 children of every parent, with no LayerNorm or
+// residual.  BF16: where it would run the 64-row halo kernel (the BF16 output's
+// rounding hides the folding's); FP32: as three BF16 terms, 1.  What the map
+// holds is checked on the device.
 int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_in, int64_t n_out,
-                   bool residual, bool y_bf16) {
-    if (!p.mfma || p.linear || !p.tl || p.tl->id != 21 || p.half_chunk || p.xf || conv->dtype != S3DX_BF16 ||
-        src.shift != 3 || !conv->pre_scale || conv->ln || residual || !y_bf16 || n_out != 8 * n_in ||
-        conv->cout % 32 != 0 || !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING"))
-        return 0;
-    const int blocks = conv->cout_pad / 32;
-    if (fold_weight_bytes(conv->cin, blocks) >= (int64_t(1) << 31) ||
+                   bool residual, int32_t y_dtype) {
+    if (!p.mfma || p.linear || !p.tl || p.xf || conv->kvol != kMaxKvol || src.shift != 3 || !conv->pre_scale ||
+        conv->ln || residual || y_dtype != conv->dtype || n_out != 8 * n_in || conv->cout % 32 != 0 ||
+        !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING") || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
         (n_in + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31))
         return 0;
+    const int blocks = conv->cout_pad / 32;
+    if (conv->dtype == S3DX_F32) {
+        if (!f3_shape(conv) || !conv->w3 || f3_fold_weight_bytes(conv->cin, conv->cout_pad) >= (int64_t(1) << 31))
+            return 0;
+        // In microseconds, as in f3_blocks: 64 parents' 8 slots of 32 columns a
+        // workgroup, 7 per chunk.
+        const int64_t passes = ((n_in + 127) / 128 * 2 * blocks + device_cus() - 1) / device_cus();
+        const double fold = 25.0 + static_cast<double>(passes) * (8.0 + 7.0 * (conv->cin / 32));
+        return fold < 4.0 + 54.0 * static_cast<double>(n_out) * conv->cin * conv->cout_pad / 95e6 ? 1 : 0;
+    }
+    if (p.tl->id != 21 || p.half_chunk || fold_weight_bytes(conv->cin, blocks) >= (int64_t(1) << 31)) return 0;
     return fold_blocks(conv->cin, blocks, p.nb, n_in, device_cus());
 }
 
@@ -822,6 +905,15 @@ void *layer_buffer(void *&buf, int64_t &have, int64_t bytes, hipStream_t s) {
         have = bytes;
     }
     return buf;
+}
+
+// The layer's buffer for what a run makes of its map: the fold state's words,
+// zeroed when the buffer is new, then `bytes` from the first KiB on.
+char *map_buffer(const s3dx_conv *conv, int64_t bytes, hipStream_t s) {
+    const int64_t had = conv->fold_bytes;
+    layer_buffer(conv->fold, conv->fold_bytes, 1024 + bytes, s);
+    if (conv->fold_bytes != had) fill_u32(static_cast<uint32_t *>(conv->fold), kFoldList, 0u, s);
+    return static_cast<char *>(conv->fold) + 1024;
 }
 
 // The layer's transformed-input buffer.
@@ -978,6 +1070,29 @@ S3DX_API s3dx_status s3dx_conv_set_weights(s3dx_conv *conv, const float *host_we
             }
             conv->w_split = ds;
         }
+        // FP32 3x3x3 layers: the three BF16 terms, split on the device from the
+        // packed weights.  Without room for them, or with a weight that has no
+        // finite terms, the layer keeps to FP32 matrix instructions.
+        if (conv->w3) (void)hipFree(conv->w3);
+        conv->w3 = nullptr;
+        if (f3_shape(conv)) {
+            const int64_t bytes = f3_weight_bytes(cin, conv->cout_pad);
+            void *d3 = nullptr;
+            if (hipMalloc(&d3, static_cast<size_t>(bytes) + 16) != hipSuccess) {
+                (void)hipGetLastError();
+            } else {
+                uint32_t *bad = reinterpret_cast<uint32_t *>(static_cast<char *>(d3) + bytes), none = 1;
+                fill_u32(bad, 1, 0u, nullptr);
+                launch_f3_weights(conv->w, d3, cin, conv->cout_pad, bad, nullptr);
+                const hipError_t e3 = hipMemcpy(&none, bad, 4, hipMemcpyDeviceToHost);
+                if (e3 != hipSuccess || none != 0) {
+                    (void)hipFree(d3);
+                    hip_check(e3, "hipMemcpy weight terms");
+                } else {
+                    conv->w3 = d3;
+                }
+            }
+        }
         replace(conv->bias, upload_f32(host_bias, static_cast<size_t>(cout)));
         conv->weights_set = true;
     });
@@ -1083,13 +1198,15 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
         LaunchPlan p = plan_launch(conv, x_bytes, n_out, true, bf16_rows);
         const bool widen = bf16_rows && !p.linear;
         if (widen) p = plan_launch(conv, src.rows * conv->cin * 4, n_out, true);
+        if (!gplan) f3_own_plan(conv, p, src, n_out);
         if (gplan) {
             require(gplan->n_out == n_out && gplan->n_src == src.n_src && gplan->shift == src.shift,
                     "gather plan was built for another map size or source rows");
-            apply_gather_plan(p, gplan, n_out, bf16_rows, conv->cin);
+            apply_gather_plan(p, conv, gplan, n_out, bf16_rows);
         }
         const bool planned = gplan && (p.fn == pick_halo_bf16_planned(64) || p.fn == pick_halo_bf16_planned(128) ||
-                                       p.fn == pick_halo_bf16_planned(64, 3) || p.stream_k);
+                                       p.fn == pick_halo_bf16_planned(64, 3) || p.f3 ||
+                                       (p.stream_k && !p.sk_splitk));
         char text[256];
         const bool halo = p.mfma && !p.linear && p.tl->id >= 20 && p.tl->id <= 22;  // the halo-staged kernels
         char groups[16] = "";
@@ -1101,9 +1218,9 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
                           p.split ? " terms=3" : "", conv->ln ? "separate" : "none", p.grid.x, groups);
         else if (p.mfma)
             std::snprintf(text, sizeof(text), "mfma tiling=%d%s%s%s rows=%d cols=%d kc=%d%s xf=%d ln=%s grid=%ux%u",
-                          p.tl->id, p.tl->splitk ? " split-k" : "", halo ? " halo" : "",
+                          p.tl->id, p.f3 ? " terms=3" : p.tl->splitk ? " split-k" : "", halo ? " halo" : "",
                           p.stream_k ? " stream-k" : "", p.tl->rows(),
-                          halo ? p.nb * 32 : p.tl->cols(), p.kc, p.half_chunk ? "+32" : "",
+                          halo || p.f3 ? p.nb * 32 : p.tl->cols(), p.kc, p.half_chunk ? "+32" : "",
                           p.xf ? 1 : 0, conv->ln ? (p.fused_ln ? "fused" : "separate") : "none", p.grid.x,
                           p.grid.y);
         else
@@ -1166,21 +1283,19 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
                           aligned(conv->pre_scale, 16) && aligned(conv->pre_shift, 16);
         LaunchPlan plan = plan_launch(conv, x_bytes, n_out, aligned16, bf16_rows,
                                       residual == nullptr && y_dtype == S3DX_BF16);
-        int fold = xvec ? fold_blocks_of(conv, plan, src, n_in, n_out, residual != nullptr, y_dtype == S3DX_BF16) : 0;
+        int fold = xvec ? fold_blocks_of(conv, plan, src, n_in, n_out, residual != nullptr, y_dtype) : 0;
         uint32_t *fold_state = nullptr, *fold_bad = nullptr;
         void *fold_records = nullptr;
         if (fold) {
             const int64_t tiles = (n_in + 127) / 128;
-            const int64_t words = static_cast<int64_t>(round_up((kFoldList + tiles) * 4, 1024));
-            const int64_t fw = fold_weight_bytes(conv->cin, conv->cout_pad / 32);
-            const int64_t had = conv->fold_bytes;
+            const int64_t list = static_cast<int64_t>(round_up((kFoldList + tiles) * 4, 1024)) - 1024;
+            const int64_t fw = bf ? fold_weight_bytes(conv->cin, conv->cout_pad / 32)
+                                  : f3_fold_weight_bytes(conv->cin, conv->cout_pad);
             try {
-                fold_state = static_cast<uint32_t *>(
-                    layer_buffer(conv->fold, conv->fold_bytes, words + tiles * kGatherPlanRecord128, s));
+                fold_records = map_buffer(conv, list + tiles * kGatherPlanRecord128, s) + list;
                 if (!conv->w_fold) hip_check(hipMalloc(&conv->w_fold, static_cast<size_t>(fw) + 16), "hipMalloc");
-                fold_records = reinterpret_cast<char *>(fold_state) + words;
+                fold_state = static_cast<uint32_t *>(conv->fold);
                 fold_bad = reinterpret_cast<uint32_t *>(static_cast<char *>(conv->w_fold) + fw);
-                if (conv->fold_bytes != had) fill_u32(fold_state, kFoldList, 0u, s);
             } catch (const oom_error &) {  // no room for the folding's buffers: the general kernel
                 (void)hipGetLastError();
                 fold_state = nullptr;
@@ -1249,29 +1364,51 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             require(gplan->n_out == n_out && gplan->n_src == src.n_src && gplan->shift == src.shift,
                     "gather plan was built for another map size or source rows");
             // Only the halo kernels read plans; other launches ignore it.
-            apply_gather_plan(plan, gplan, n_out, bf16_rows, conv->cin);
+            apply_gather_plan(plan, conv, gplan, n_out, bf16_rows);
             if (plan.fn == pick_halo_bf16_planned(64) || plan.fn == pick_halo_bf16_planned(128) ||
-                plan.fn == pick_halo_bf16_planned(64, 3) || plan.stream_k)
+                plan.fn == pick_halo_bf16_planned(64, 3) || plan.f3 || plan.stream_k)
                 a.plan = gplan->d;
+            a.w3 = conv->w3;
         }
         if (fold) {
             if (!conv->w_fold_ready) {
                 fill_u32(fold_bad, 1, 0u, s);
-                launch_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad / 32, fold_bad, s);
+                if (bf) launch_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad / 32, fold_bad, s);
+                else launch_f3_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad, fold_bad, s);
                 launch_check("fold_weights");
                 conv->w_fold_ready = true;
             }
-            launch_fold_plan(kmap, n_in, fold_records, fold_state, fold_bad, s);
+            launch_fold_plan(kmap, n_in, fold_records, fold_state, fold_bad, !bf, s);
             launch_check("fold_plan");
             ConvArgs fa = a;
-            fa.w = conv->w_fold;
             fa.plan = fold_records;
+            if (!bf) {
+                fa.w3 = conv->w_fold;
+                launch_conv_f3_fold(fa, fold_state, s);
+                return;
+            }
+            fa.w = conv->w_fold;
             launch_conv_fold(fa, fold, s);
             launch_check("conv_fold");
             a.plan = nullptr;
             launch_halo_listed(a, plan.nb, fold_state, s);
             launch_check("conv_halo_listed");
             return;
+        }
+        if (!gplan && aligned16) {
+            const LaunchPlan whole = plan;
+            if (f3_own_plan(conv, plan, src, n_out)) {
+                try {
+                    void *records = map_buffer(conv, (n_out + 127) / 128 * kGatherPlanRecord128, s);
+                    launch_gather_plan_build(128, kmap, n_out, src.n_src, src.shift, records, s);
+                    launch_check("gather_plan_build");
+                    a.plan = records;
+                    a.w3 = conv->w3;
+                } catch (const oom_error &) {
+                    (void)hipGetLastError();
+                    plan = whole;
+                }
+            }
         }
         // A LayerNorm the epilogue cannot fuse runs as its own pass over the
         // conv's FP32 output (the layer's buffer), then modulate, SiLU and
@@ -1346,6 +1483,7 @@ void gather_plan_build(s3dx_gather_plan *p, const s3dx_conv *conv, int64_t n_in,
     p->n_out = n_out;
     p->n_src = src.n_src;
     p->shift = src.shift;
+    p->f32 = conv->dtype == S3DX_F32;
 }
 
 void gather_plan_check(const s3dx_conv *conv, int64_t n_in, const int32_t *kmap, int64_t n_out) {
@@ -1410,6 +1548,7 @@ S3DX_API s3dx_status s3dx_kmap_subm3_planned(const int32_t *coords, int64_t n, i
         plan->n_out = n;
         plan->n_src = n;
         plan->shift = 0;
+        plan->f32 = conv->dtype == S3DX_F32;
     });
 }
 

@@ -114,7 +114,7 @@ struct FoldSlice {
 
 __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const int32_t *kmap, int64_t n_parents,
                                                                          char *plan, uint32_t *state,
-                                                                         const uint32_t *bad_weights) {
+                                                                         const uint32_t *bad_weights, int most) {
     // A parent's 8 * 27 child entries are 54 16-byte pieces; 864 of the threads
     // take the pieces of 16 parents a pass, each thread the same piece of
     // every parent, so that what its four entries are (the parent offset they
@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const i
     const TileDedupe dd = plan_tile<4, NTH>(FoldSlice{parents}, n_parents, n_parents, 0, plan);
     // (plan_tile's barriers order the writes of `wrong` before this read, and
     // thread 0 wrote the record's header)
-    if (tid == 0 && (wrong != 0u || dd.global_a || dd.distinct > static_cast<uint32_t>(kH8Double))) {
+    if (tid == 0 && (wrong != 0u || dd.global_a || dd.distinct > static_cast<uint32_t>(most))) {
         *reinterpret_cast<uint32_t *>(plan + static_cast<int64_t>(tile) * kGatherPlanRecord128) = kFoldGeneral;
         const uint32_t at = atomicAdd(state + kFoldCount, 1u);
         state[kFoldList + at] = static_cast<uint32_t>(tile);
@@ -449,10 +449,10 @@ void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t
 }
 
 void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
-                      hipStream_t stream) {
+                      bool f32, hipStream_t stream) {
     hipLaunchKernelGGL(fold_plan_kernel, dim3(static_cast<unsigned>((n_parents + 127) / 128)),
                        dim3(kPlanBuild128Threads), 0, stream, kmap, n_parents, static_cast<char *>(plan), state,
-                       bad_weights);
+                       bad_weights, f32 ? kF3MostRows : kH8Double);
 }
 
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream) {

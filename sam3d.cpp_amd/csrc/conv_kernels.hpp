@@ -34,6 +34,7 @@ struct ConvArgs {
     const float *mod_shift;
     int32_t silu;
     const void *plan;  // per-tile gather plan records (halo kernel), or nullptr
+    const void *w3;    // FP32 layers on BF16 matrix units: the weights' three terms
     // Stream-K launches of the 8-wave halo kernel: sk_wgs equal runs over the
     // sk_units (column group, tile, chunk) units, and two FP32 128 x 128 tile
     // slots per run for the pieces that are part of a tile.
@@ -47,7 +48,8 @@ using KernelFn = void (*)(ConvArgs);
 // Workgroup tilings of the MFMA kernel: 4 waves in WM x WN (WM = 4/WN), each
 // wave MBW x NBW blocks of 32x32 outputs.
 // Tilings 20, 21: the halo-staged kernel (conv_halo.hip), 128- and 64-row split-K tiles;
-// 22: its 8-wave 128-row variant, launched only with a 128-row gather plan.
+// 22: its 8-wave 128-row variant, launched only with a 128-row gather plan;
+// 25: FP32 layers as three BF16 terms (conv_f3.hip), the same.
 // Split-K tilings (splitk = 1): 128 rows x 32*nbw columns, each wave owning
 // the whole tile for a quarter of the k-steps.  Ids 15 and 16 (BF16, 32- or
 // 64-channel chunks) build each 128-channel task from 4 or 2 chunks.  Ids 17
@@ -65,6 +67,7 @@ inline constexpr Tiling kTilings[] = {
     {15, 4, 3, 1, 1}, {16, 4, 4, 1, 1}, {18, 2, 4, 1, 1},
     {19, 2, 3, 1, 1}, {20, 4, 4, 1, 1}, {21, 2, 4, 1, 1}, {22, 4, 4, 1, 1},
     {23, 2, 1, 1, 1}, {24, 1, 1, 1, 1},
+    {25, 4, 4, 1, 1},
 };
 
 // MFMA kernel for tiling `id`, kc channels per task, xf 64-bit gathers;
@@ -107,6 +110,19 @@ void launch_kmap_plan(int rows, const int32_t *coords, int64_t n, int32_t missin
                       uint64_t workspace_bytes, void *plan, hipStream_t stream);
 constexpr int kGatherPlanRecord = 7168;      // 64-row tiles
 constexpr int kGatherPlanRecord128 = 18432;  // 128-row tiles
+// FP32 layers as three BF16 terms (conv_f3.hip): the weights' terms from the
+// packed FP32 ones (*bad: raised when one has no finite terms), and the kernel
+// for 128-row plan records and cg 32-column blocks per workgroup (4, 2, 1),
+// launched with kHalo8Threads threads.
+int64_t f3_weight_bytes(int cin, int cout_pad);
+void launch_f3_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
+KernelFn pick_f3(int cg);
+constexpr int kF3MostRows = 719;  // distinct rows of a tile that it stages
+// The same for folded parent rows: the folded weights' terms, and the folded
+// run with the FP32 pass over the listed tiles behind it.
+int64_t f3_fold_weight_bytes(int cin, int cout_pad);
+void launch_f3_fold_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
+void launch_conv_f3_fold(const ConvArgs &a, uint32_t *state, hipStream_t stream);
 // Folded convs over repeated parent rows (conv_fold.hip).  `state`: the words
 // below, then the list (one word per 128 parents); the count is cleared before
 // each run's plan, the flag by the listed pass that ends a run.
@@ -119,7 +135,7 @@ int fold_blocks(int cin, int blocks, int general_nb, int64_t n_parents, int64_t 
 // *bad: raised when a folded weight is no finite number.
 void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t *bad, hipStream_t stream);
 void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
-                      hipStream_t stream);
+                      bool f32, hipStream_t stream);
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
 // The general kernel (64-row tiles, nb column blocks) over the listed tiles.
 void launch_halo_listed(const ConvArgs &a, int nb, uint32_t *state, hipStream_t stream);

@@ -1,0 +1,219 @@
+"""FP32 3x3x3 convs as three BF16 terms (conv_f3.hip).
+
+With a gather plan made for an FP32 layer (or, in a layer with input
+transforms, records of its own) the six term products above 2^-27 of each
+product are accumulated in FP32.  Their error against float64 must not exceed
+the FP32 matrix instructions' on the same inputs (measured: a quarter to nine
+tenths of it), and the FP32 gate (rel-L2 1e-5) holds far off.  Rows in LDS (up
+to 719 distinct ones in a tile), rows gathered from memory, and infinities or
+NaN, which take FP32 matrix instructions, are all reached.
+"""
+import numpy as np
+import pytest
+
+from helpers import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(x, kmap, w, b, mesh=False):
+    """float64 sum over the offsets; w [cout][27][cin], or [27][cout][cin]."""
+    w = np.asarray(w, np.float64).transpose(1, 0, 2) if not mesh else np.asarray(w, np.float64)
+    y = np.tile(np.asarray(b, np.float64), (kmap.shape[0], 1))
+    for o in range(27):
+        at = np.flatnonzero((kmap[:, o] >= 0) & (kmap[:, o] < x.shape[0]))
+        y[at] += x[kmap[at, o]].astype(np.float64) @ w[o].T
+    return y
+
+
+def _regions(c, runs):
+    """Rows so that each 128 of them come from `runs` places of the set."""
+    n = c.shape[0] // 128 * 128
+    step = 128 // runs
+    idx = np.arange(n).reshape(runs, -1, step).transpose(1, 0, 2).reshape(-1)
+    return np.ascontiguousarray(c[idx])
+
+
+def _points(step):
+    g = np.stack(np.meshgrid(*(np.arange(0, 60, step),) * 3, indexing="ij"), -1).reshape(-1, 3)
+    return np.ascontiguousarray(np.concatenate([np.zeros((len(g), 1), np.int64), g], 1).astype(np.int32))
+
+
+def _shuffled(c):
+    return np.ascontiguousarray(c[np.random.default_rng(5).permutation(len(c))])
+
+
+CASES = {
+    # name: (coords, cin, cout, LayerNorm, columns a workgroup)
+    "whole_row_ln": (lambda W: W.shells_union(0)[:12801], 128, 128, True, 128),
+    "two_blocks": (lambda W: W.shells_union(0)[:9000], 64, 192, False, 64),
+    "one_block_ragged_cout": (lambda W: W.shells_union(1)[:6007], 128, 90, False, 32),
+    "wide_separate_ln": (lambda W: W.shells_union(2)[:6001], 96, 256, True, None),
+    "two_places": (lambda W: _regions(W.shells_union(0)[:12800], 2), 64, 128, False, None),    # 560 to 719 rows
+    "four_places": (lambda W: _regions(W.shells_union(0)[:12800], 4), 64, 128, False, None),   # around 719
+    "eight_places": (lambda W: _regions(W.shells_union(0)[:12800], 8), 96, 64, False, None),   # above: from memory
+    "shuffled": (lambda W: _shuffled(W.shells_union(0)[:12000]), 64, 128, False, None),        # the plan's global tiles
+    "isolated_points": (lambda W: _points(3), 128, 128, False, None),                          # one offset
+}
+
+
+def _layer(s3dx, W, cin, cout, ln, seed=90):
+    w, b = W.conv_weight(seed, 2, cin, cout), W.normal_f32(seed, 3, (cout,), 0.1)
+    conv = s3dx.SparseConv(cin, cout, 27, s3dx.F32).set_weights(w, s3dx.WEIGHT_SLAT, b)
+    if ln:
+        conv.set_layernorm(True, 1e-6).set_silu(True)
+    return conv, w, b
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_error_no_larger_than_fp32(s3dx, O, W, name):
+    make, cin, cout, ln, cols = CASES[name]
+    coords = make(W)
+    n = coords.shape[0]
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, b = _layer(s3dx, W, cin, cout, ln)
+    x, res = W.normal_f32(90, 1, (n, cin)), W.normal_f32(90, 4, (n, cout))
+    xd, kd, rd = (s3dx.DeviceArray.from_host(a) for a in (x, kmap, res))
+    gp = conv.gather_plan(n, kd, n)
+    text = conv.plan(n, n, gp)
+    print(f"{name}: n={n} {cin}->{cout}: {text}", flush=True)
+    assert text.startswith("mfma tiling=25 terms=3 rows=128") and text.endswith(" plan=128"), text
+    assert cols is None or f" cols={cols} " in text, text
+    ys = [s3dx.DeviceArray((n, cout), np.float32) for _ in range(3)]
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32, rd, plan=gp)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32, rd, plan=gp)
+    conv.run(xd, n, kd, n, ys[2], s3dx.F32, rd)  # FP32 matrix instructions
+    got, again, fp32 = (y.download() for y in ys)
+    assert np.array_equal(got, again), "two runs differ"
+    ref = _ref(x, kmap, w, b)
+    if ln:
+        ref = (ref - ref.mean(1, keepdims=True)) / np.sqrt(ref.var(1, keepdims=True) + 1e-6)
+        ref = ref / (1.0 + np.exp(-ref))
+    ref += res
+    e, f = rel_l2(got, ref), rel_l2(fp32, ref)
+    print(f"  rel-L2 three terms {e:.2e}, FP32 {f:.2e}", flush=True)
+    assert e <= 1.05 * f and e < 1e-6, (e, f)
+    worst = np.max(np.abs(got - ref)) / np.max(np.abs(ref))
+    assert worst < 4e-6, worst
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** 100])
+def test_scales(s3dx, O, W, scale):
+    # The terms keep FP32's exponent range.
+    coords = W.shells_union(0)[:9000]
+    n = coords.shape[0]
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, _ = _layer(s3dx, W, 64, 128, False)
+    conv.set_weights(w, s3dx.WEIGHT_SLAT, None)
+    x = W.normal_f32(91, 1, (n, 64))
+    kd = s3dx.DeviceArray.from_host(kmap)
+    gp = conv.gather_plan(n, kd, n)
+    y = s3dx.DeviceArray((n, 128), np.float32)
+    conv.run(s3dx.DeviceArray.from_host((x * np.float32(scale)).astype(np.float32)), n, kd, n, y, s3dx.F32, plan=gp)
+    assert rel_l2(y.download().astype(np.float64) / scale, _ref(x, kmap, w, np.zeros(128))) < 1e-6
+
+
+@pytest.mark.parametrize("places", [1, 8])
+def test_infinities_nan_and_large_values(s3dx, O, W, places):
+    coords = _regions(W.shells_union(0)[:9088], places)
+    n = coords.shape[0]
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, b = _layer(s3dx, W, 64, 128, False)
+    x = W.normal_f32(92, 1, (n, 64))
+    clean = x.copy()
+    x[500, 3], x[3000, 9], x[3000, 10], x[6000, 1] = np.inf, -np.inf, np.inf, np.nan
+    x[8000, 5] = np.finfo(np.float32).max  # its first term would be infinite
+    kd = s3dx.DeviceArray.from_host(kmap)
+    gp = conv.gather_plan(n, kd, n)
+    ys = [s3dx.DeviceArray((n, 128), np.float32) for _ in range(3)]
+    xd = s3dx.DeviceArray.from_host(x)
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32, plan=gp)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32)
+    conv.run(s3dx.DeviceArray.from_host(clean), n, kd, n, ys[2], s3dx.F32, plan=gp)
+    got, want, ok = (y.download() for y in ys)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want)) and np.isinf(want).any() and np.isnan(want).any()
+    fin = np.isfinite(want)
+    assert np.all(np.abs(got[fin].astype(np.float64) - want[fin]) <= 1e-5 * np.maximum(1.0, np.abs(want[fin].astype(np.float64))))
+    assert np.isfinite(ok).all()
+
+
+def test_weights_without_terms(s3dx, O, W):
+    # An infinite weight: the layer keeps to FP32 matrix instructions.
+    coords = W.shells_union(0)[:9000]
+    n = coords.shape[0]
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, b = _layer(s3dx, W, 64, 128, False)
+    w[3, 13, 5] = np.inf
+    conv.set_weights(w, s3dx.WEIGHT_SLAT, b)
+    kd = s3dx.DeviceArray.from_host(kmap)
+    gp = conv.gather_plan(n, kd, n)
+    assert "terms=3" not in conv.plan(n, n, gp)
+    xd = s3dx.DeviceArray.from_host(W.normal_f32(93, 1, (n, 64)))
+    ys = [s3dx.DeviceArray((n, 128), np.float32) for _ in range(2)]
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32, plan=gp)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32)
+    assert np.array_equal(ys[0].download(), ys[1].download(), equal_nan=True)
+
+
+def _mesh(s3dx, W, p, cin, cout, parent, seed=95):
+    parents = W.shells_union(0)[:p]
+    _, kd = s3dx.subdivide2(s3dx.DeviceArray.from_host(parents), p, True)
+    rows = p if parent else 8 * p
+    x = W.normal_f32(seed, 1, (rows, cin))
+    scale, shift = W.normal_f32(seed, 2, (cin,), 0.2) + 1.0, W.normal_f32(seed, 3, (cin,), 0.2)
+    w, b = W.conv_weight(seed, 4, cin, cout, layout="mesh"), W.normal_f32(seed, 5, (cout,), 0.1)
+    conv = (s3dx.SparseConv(cin, cout, 27, s3dx.F32).set_weights(w, s3dx.WEIGHT_MESH, b).set_gather_parent(parent)
+            .set_input_affine_silu(s3dx.DeviceArray.from_host(scale), s3dx.DeviceArray.from_host(shift)))
+    v = x.astype(np.float64) * scale + shift
+    return conv, kd.download(), x, (v / (1.0 + np.exp(-v))), w, b
+
+
+def _run(s3dx, conv, x, kmap, cout):
+    y = s3dx.DeviceArray((kmap.shape[0], cout), np.float32)
+    conv.run(s3dx.DeviceArray.from_host(x), x.shape[0], s3dx.DeviceArray.from_host(kmap), kmap.shape[0], y, s3dx.F32)
+    return y.download()
+
+
+@pytest.mark.parametrize("p,cin,cout,parent", [
+    (3001, 192, 96, True),    # folded, a ragged last tile
+    (1500, 64, 128, True),
+    (2003, 96, 96, False),    # the map's records built in the run
+    (1100, 192, 192, False),
+])
+def test_layers_with_transforms(s3dx, W, monkeypatch, p, cin, cout, parent):
+    conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, parent)
+    print(f"p={p} {cin}->{cout} parent={parent}: {conv.plan(x.shape[0], 8 * p)}", flush=True)
+    got = _run(s3dx, conv, x, kmap, cout)
+    assert np.array_equal(got, _run(s3dx, conv, x, kmap, cout)), "two runs differ"
+    monkeypatch.setenv("S3DX_CONV_TILING", "11")
+    fp32 = _run(s3dx, conv, x, kmap, cout)
+    monkeypatch.delenv("S3DX_CONV_TILING")
+    assert not np.array_equal(got, fp32)  # (the FP32 kernel, that is)
+    km = np.where(kmap >= 0, kmap >> 3, -1) if parent else kmap
+    ref = _ref(h, km, w, b, mesh=True)
+    e, f = rel_l2(got, ref), rel_l2(fp32, ref)
+    print(f"  rel-L2 {e:.2e}, FP32 {f:.2e}", flush=True)
+    assert e <= 1.05 * f and e < 2e-6, (e, f)
+
+
+def test_folded_fp32_maps_and_infinities(s3dx, W, monkeypatch):
+    # Tiles no subdivide made, and rows with an infinity, run FP32 matrix
+    # instructions: near the FP32 kernel's values, the same infinities and NaN.
+    p, cin, cout = 3001, 64, 96
+    conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, True)
+    bad = kmap.copy()
+    bad[8 * 130 + 3, 14] = -1
+    bad[8 * 300, 26] = 8 * 2000 + 1
+    bad[8 * 1500:8 * 1600] = np.random.default_rng(2).integers(-1, 8 * p, (800, 27), dtype=np.int32)
+    for m in (bad, np.full_like(kmap, -1)):
+        assert rel_l2(_run(s3dx, conv, x, m, cout), _ref(h, np.where(m >= 0, m >> 3, -1), w, b, mesh=True)) < 2e-6
+    xi = x.copy()
+    xi[700, 3], xi[900, 1] = np.inf, np.nan
+    got = _run(s3dx, conv, xi, kmap, cout)
+    monkeypatch.setenv("S3DX_CONV_TILING", "11")
+    want = _run(s3dx, conv, xi, kmap, cout)
+    monkeypatch.delenv("S3DX_CONV_TILING")
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and np.isnan(want).any()
+    first = _run(s3dx, conv, x, kmap, cout)
+    assert rel_l2(first, _ref(h, np.where(kmap >= 0, kmap >> 3, -1), w, b, mesh=True)) < 2e-6
