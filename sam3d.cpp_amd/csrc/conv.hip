@@ -879,6 +879,21 @@ int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src
     return fold_blocks(conv->cin, blocks, p.nb, n_in, device_cus());
 }
 
+// Whether a run goes by 512-row tiles (conv_rows.hip): an unplanned BF16 layer
+// with an input affine (so with buffers of its own) that no halo kernel suits
+// (Cin 32 above a multiple of 64), 96-column groups, BF16 output and no
+// LayerNorm, over at least as many tiles as CUs (96 -> 96 on 256,000 rows: 176
+// against 225 us; below, the 64-row tiles fill the GPU better).
+bool rows_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_out, int32_t y_dtype) {
+    return p.mfma && !p.linear && p.tl && p.tl->id != 20 && p.tl->id != 21 && !p.xf && conv->kvol == kMaxKvol &&
+           conv->dtype == S3DX_BF16 && conv->pre_scale && src.shift == 0 && !conv->ln && y_dtype == S3DX_BF16 &&
+           conv->cin % 32 == 0 && conv->cout % 96 == 0 && aligned(conv->bias, 16) &&
+           !std::getenv("S3DX_CONV_TILING") && !std::getenv("S3DX_CONV_HALO") &&
+           n_out * kMaxKvol * 4 < (int64_t(1) << 31) && (n_out + 511) / 512 * int64_t(kRowsRecord) < (int64_t(1) << 31) &&
+           int64_t(kMaxKvol) * conv->cin * conv->cout_pad * 2 < (int64_t(1) << 31) &&
+           (n_out + 511) / 512 * (conv->cout / 96) >= device_cus();
+}
+
 float *upload_f32(const float *host, size_t count) {
     if (!host) return nullptr;
     void *d = nullptr;
@@ -1302,6 +1317,18 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
                 fold = 0;
             }
         }
+        // Runs by 512-row tiles: the same state words, its records behind the list.
+        const int64_t row_tiles = (n_out + 511) / 512;
+        const int64_t row_list = static_cast<int64_t>(round_up((kFoldList + row_tiles) * 4, 1024)) - 1024;
+        char *row_records = nullptr;
+        if (!gplan && xvec && aligned16 && rows_of(conv, plan, src, n_out, y_dtype)) {
+            try {
+                row_records = map_buffer(conv, row_list + row_tiles * kRowsRecord, s) + row_list;
+                fold_state = static_cast<uint32_t *>(conv->fold);
+            } catch (const oom_error &) {
+                (void)hipGetLastError();
+            }
+        }
         if (src.pre) {
             XformArgs xa{};
             xa.fold_state = fold_state;
@@ -1391,7 +1418,18 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             launch_conv_fold(fa, fold, s);
             launch_check("conv_fold");
             a.plan = nullptr;
-            launch_halo_listed(a, plan.nb, fold_state, s);
+            launch_halo_listed(a, plan.nb, 16, fold_state, s);
+            launch_check("conv_halo_listed");
+            return;
+        }
+        if (row_records) {
+            launch_rows_plan(kmap, n_out, src.n_src, row_records, fold_state, s);
+            launch_check("rows_plan");
+            ConvArgs ra = a;
+            ra.plan = row_records;
+            launch_conv_rows(ra, s);
+            launch_check("conv_rows");
+            launch_halo_listed(a, 3, 8, fold_state, s);
             launch_check("conv_halo_listed");
             return;
         }

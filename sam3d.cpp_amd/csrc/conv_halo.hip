@@ -356,14 +356,15 @@ __global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_halo_kernel(ConvArg
     halo_body<MB, PLAN, NB>(a, xcd_tile(blockIdx.x, gridDim.x), blockIdx.y * NB);
 }
 
-// The 64-row tiles of the parent tiles that a folded run left over (128
-// parents: 16 tiles), by however many workgroups there are; usually none.
+// The 64-row tiles of the larger tiles (per of them each) that a folded run,
+// or one by 512-row tiles, left over, by however many workgroups there are;
+// usually none.
 template <int NB>
-__global__ void __launch_bounds__(256, 1) conv_halo_listed_kernel(ConvArgs a, uint32_t *state) {
-    const int64_t total = static_cast<int64_t>(state[kFoldCount]) * 16;
+__global__ void __launch_bounds__(256, 1) conv_halo_listed_kernel(ConvArgs a, int per, uint32_t *state) {
+    const int64_t total = static_cast<int64_t>(state[kFoldCount]) * per;
     const int64_t tiles = (a.n_out + 63) / 64;
     for (int64_t i = blockIdx.x; i < total; i += gridDim.x) {
-        const int64_t tile = static_cast<int64_t>(state[kFoldList + i / 16]) * 16 + i % 16;
+        const int64_t tile = static_cast<int64_t>(state[kFoldList + i / per]) * per + i % per;
         if (tile >= tiles) continue;
         __syncthreads();  // the previous tile is done with LDS
         halo_body<2, false, NB>(a, static_cast<int>(tile), blockIdx.y * NB);
@@ -1117,11 +1118,11 @@ KernelFn pick_halo_bf16(int rows, int nb) {
     return rows == 128 ? conv_halo_kernel<4, false> : rows == 64 ? conv_halo_kernel<2, false> : nullptr;
 }
 
-void launch_halo_listed(const ConvArgs &a, int nb, uint32_t *state, hipStream_t stream) {
+void launch_halo_listed(const ConvArgs &a, int nb, int per, uint32_t *state, hipStream_t stream) {
     const unsigned tiles = static_cast<unsigned>(std::min<int64_t>((a.n_out + 63) / 64, 512));
     const dim3 grid(tiles, static_cast<unsigned>(a.cout_pad / 32 / nb));
-    if (nb == 3) hipLaunchKernelGGL(conv_halo_listed_kernel<3>, grid, dim3(256), 0, stream, a, state);
-    else hipLaunchKernelGGL(conv_halo_listed_kernel<4>, grid, dim3(256), 0, stream, a, state);
+    if (nb == 3) hipLaunchKernelGGL(conv_halo_listed_kernel<3>, grid, dim3(256), 0, stream, a, per, state);
+    else hipLaunchKernelGGL(conv_halo_listed_kernel<4>, grid, dim3(256), 0, stream, a, per, state);
 }
 
 KernelFn pick_halo8_stream_k() { return conv_halo8_sk_kernel; }

@@ -137,8 +137,15 @@ void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t
 void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
                       bool f32, hipStream_t stream);
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
-// The general kernel (64-row tiles, nb column blocks) over the listed tiles.
-void launch_halo_listed(const ConvArgs &a, int nb, uint32_t *state, hipStream_t stream);
+// The general kernel (64-row tiles, nb column blocks) over the listed tiles of
+// `per` * 64 rows.
+void launch_halo_listed(const ConvArgs &a, int nb, int per, uint32_t *state, hipStream_t stream);
+// BF16 convs over many rows, 96 columns a workgroup (conv_rows.hip): a record
+// per 512 rows, and the state words above for the tiles left to the general
+// kernel.
+constexpr int kRowsRecord = 34816;
+void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, uint32_t *state, hipStream_t stream);
+void launch_conv_rows(const ConvArgs &a, hipStream_t stream);
 // The FP32 1x1-layer kernel reading BF16 rows, else nullptr.
 KernelFn pick_linear_f32_bf16_rows(int nbt);
 // The same on BF16 MFMAs with three-term split weights (Cin = 16 * ksx,

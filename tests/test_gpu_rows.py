@@ -1,0 +1,60 @@
+"""BF16 convs by 512-row tiles (conv_rows.hip): Cin 96 over many rows, the mesh
+decoder's last conv.  Against the split-K kernel (S3DX_CONV_TILING=19): both
+accumulate in FP32 and round once to BF16, in different orders, so the outputs
+differ by one BF16 step here and there (rel-L2 far below 2^-9).  Tiles without
+all 27 offsets, of more rows than the LDS holds, or of rows further apart than
+the plan's bitmap run the 64-row halo kernel.
+"""
+import numpy as np
+import pytest
+
+from helpers import check_rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cin,cout,residual,silu", [(96, 96, True, False), (32, 96, False, True), (160, 192, True, False)])
+def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
+    parents = W.shells_union(0)[:16421]
+    p = parents.shape[0]
+    n = 8 * p  # 257 tiles, the last of 296 rows
+    _, kd = s3dx.subdivide2(s3dx.DeviceArray.from_host(parents), p, True)
+    kmap = kd.download()
+    whole = kmap.copy()
+    kmap[512 * 3:512 * 4, 5] = -1                    # an offset that no row of the tile has
+    kmap[512 * 7 + 100, 20] = n - 1                  # a row far away
+    rng = np.random.default_rng(1)
+    kmap[512 * 9:512 * 10] = rng.integers(-1, 16000, (512, 27), dtype=np.int32)  # too many rows
+    kmap[512 * 256 + 3] = -1
+    seed = 110
+    x = W.round_bf16(W.normal_f32(seed, 1, (n, cin)))
+    scale, shift = W.normal_f32(seed, 2, (cin,), 0.2) + 1.0, W.normal_f32(seed, 3, (cin,), 0.2)
+    w, b = W.conv_weight(seed, 4, cin, cout, layout="mesh"), W.normal_f32(seed, 5, (cout,), 0.1)
+    res = W.round_bf16(W.normal_f32(seed, 6, (p, cout)))
+    conv = (s3dx.SparseConv(cin, cout, 27, s3dx.BF16).set_weights(w, s3dx.WEIGHT_MESH, b)
+            .set_input_affine_silu(s3dx.DeviceArray.from_host(scale), s3dx.DeviceArray.from_host(shift))
+            .set_residual_parent(True).set_silu(silu))
+    xd = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(x))
+    rd = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(res)) if residual else None
+
+    def run(m):
+        y = s3dx.DeviceArray((n, cout), np.uint16)
+        conv.run(xd, n, s3dx.DeviceArray.from_host(m), n, y, s3dx.BF16, rd)
+        return y.download()
+
+    a = W.round_bf16(O.silu((x * scale + shift).astype(np.float32)))
+    rows = np.unique(np.concatenate([np.sort(rng.choice(n, 1200, replace=False)), np.arange(512 * 3, 512 * 3 + 40),
+                                     [512 * 7 + 100, 512 * 9 + 5, 512 * 256 + 3, n - 1]]))
+    for name, m in (("subdivide's map", whole), ("with other tiles", kmap)):
+        got = run(m)
+        assert np.array_equal(got, run(m)), "two runs differ"
+        monkeypatch.setenv("S3DX_CONV_TILING", "19")
+        want = run(m)
+        monkeypatch.delenv("S3DX_CONV_TILING")
+        g, v = (W.bf16_bits_to_f32(t).reshape(t.shape) for t in (got, want))
+        rel = float(np.linalg.norm(g - v) / np.linalg.norm(v))
+        print(f"{cin}->{cout} {name}: rel-L2 against split-K {rel:.2e}", flush=True)
+        assert 0.0 < rel < 2.0 ** -11  # (0: the kernel did not run)
+        ref = O.conv(a, m[rows], n, W.round_bf16(w), 1, cout, b)
+        ref = O.silu(ref) if silu else ref
+        check_rel(g[rows], ref + (res[rows >> 3] if residual else 0.0), 1e-2, "oracle")
