@@ -67,9 +67,9 @@ __device__ __forceinline__ int32_t hash_find(const Hash &h, int4 c) {
     return -1;
 }
 
-// Empties the slots and zeroes the flag words (one launch for both).
-__global__ void __launch_bounds__(kThreads) hash_clear_kernel(Hash h) {
-    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+// Thread i's share of emptying the slots and zeroing the flag words (a grid
+// over mask + 1 threads; the callers' kernels prepare the keys beside it).
+__device__ __forceinline__ void hash_clear(const Hash &h, uint32_t i) {
     if (i <= h.mask) h.slots[i] = kEmpty;
     if (i < 64) h.flags[i] = 0;
 }
@@ -104,14 +104,14 @@ __device__ __forceinline__ bool add_fits(int32_t v, int32_t d, int32_t *out) {
 unsigned blocks_for(int64_t items) { return static_cast<unsigned>((items + kThreads - 1) / kThreads); }
 
 // Grid of a bounds reduction: at most 128 blocks, each thread striding over
-// the items, so the per-block atomics stay few.
+// the items.
 inline unsigned bounds_blocks(int64_t items) { return blocks_for(items) < 128u ? blocks_for(items) : 128u; }
 
-// Block-wide min of v[0..M) and max of v[M..2M), committed with one atomic
-// per value per block: a wave butterfly, then the block's waves through LDS.
-// Every thread of the block must call it.
+// Block-wide min of v[0..M) and max of v[M..2M), written to out[0..2M) by
+// one thread: a wave butterfly, then the block's waves through LDS.  Every
+// thread of the block must call it.
 template <int M>
-__device__ __forceinline__ void block_bounds_atomic(int (&v)[2 * M], int32_t *out) {
+__device__ __forceinline__ void block_bounds(int (&v)[2 * M], int32_t *out) {
     __shared__ int part[kThreads / 64][2 * M];
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -129,8 +129,7 @@ __device__ __forceinline__ void block_bounds_atomic(int (&v)[2 * M], int32_t *ou
         for (int a = 0; a < 2 * M; ++a) {
             int r = part[0][a];
             for (int w = 1; w < kThreads / 64; ++w) r = a < M ? min(r, part[w][a]) : max(r, part[w][a]);
-            if (a < M) atomicMin(&out[a], r);
-            else atomicMax(&out[a], r);
+            out[a] = r;
         }
     }
 }
@@ -155,13 +154,9 @@ void hash_layout(W &w, int64_t n, Hash *h) {
     }
 }
 
-// Clears the table and inserts n keys (first occurrence wins).
-inline void hash_build(const int4 *keys, int32_t n, Hash &h, hipStream_t stream) {
-    h.keys = keys;
-    const uint64_t cap = static_cast<uint64_t>(h.mask) + 1;
-    hash_clear_kernel<<<blocks_for(static_cast<int64_t>(cap)), kThreads, 0, stream>>>(h);
-    launch_check("hash_clear");
-    hash_insert_kernel<<<blocks_for(n), kThreads, 0, stream>>>(keys, n, h);
+// Inserts n keys into the emptied table (first occurrence wins).
+inline void hash_insert(const Hash &h, int32_t n, hipStream_t stream) {
+    hash_insert_kernel<<<blocks_for(n), kThreads, 0, stream>>>(h.keys, n, h);
     launch_check("hash_insert");
 }
 
