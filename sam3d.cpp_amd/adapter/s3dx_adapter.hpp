@@ -146,7 +146,8 @@ public:
     s3dx_conv *get() const { return c_; }
     explicit operator bool() const { return c_ != nullptr; }
     // With a gather plan of kmap (GatherPlan below) the halo kernels skip
-    // their per-tile dedupe; results are the same bits either way.
+    // their per-tile dedupe: BF16 whole tiles give the same bits either way;
+    // FP32 layers run as three BF16 terms over it, within FP32 rounding.
     void run(const void *x, int64_t n_in, const int32_t *kmap, int64_t n_out, const void *residual, void *y,
              int32_t y_dtype, s3dx_stream s, const s3dx_gather_plan *plan = nullptr) const {
         char err[512];

@@ -133,19 +133,17 @@ __device__ __forceinline__ void adjacent(int ch, int o, int *parent_offset, int 
     *child_slot = cs;
 }
 
+__device__ __forceinline__ int4 child_row(int4 c, int ch) {
+    return make_int4(c.x, static_cast<int32_t>(static_cast<uint32_t>(c.y) * 2u + static_cast<uint32_t>(ch >> 2)),
+                     static_cast<int32_t>(static_cast<uint32_t>(c.z) * 2u + static_cast<uint32_t>((ch >> 1) & 1)),
+                     static_cast<int32_t>(static_cast<uint32_t>(c.w) * 2u + static_cast<uint32_t>(ch & 1)));
+}
+
 __global__ void __launch_bounds__(kThreads)
 child_coords_kernel(const int4 *__restrict__ parents, int32_t p, int4 *__restrict__ children) {
     const int32_t r = blockIdx.x * kThreads + threadIdx.x;
     if (r >= p * 8) return;
-    const int4 c = parents[r >> 3];
-    const int ch = r & 7;
-    int4 out;
-    out.x = c.x;
-    out.y = static_cast<int32_t>(static_cast<uint32_t>(c.y) * 2u + static_cast<uint32_t>(ch >> 2));
-    out.z = static_cast<int32_t>(static_cast<uint32_t>(c.z) * 2u +
-                                 static_cast<uint32_t>((ch >> 1) & 1));
-    out.w = static_cast<int32_t>(static_cast<uint32_t>(c.w) * 2u + static_cast<uint32_t>(ch & 1));
-    children[r] = out;
+    children[r] = child_row(parents[r >> 3], r & 7);
 }
 
 // One thread per (child, offset): neighbour = parent_nbr*8 + child slot.
@@ -161,41 +159,43 @@ child_kmap_kernel(const int32_t *__restrict__ parent_kmap, int32_t p, int32_t *_
     kmap[g] = t >= 0 ? t * 8 + cs : -1;
 }
 
-// Four entries per thread (32-bit indexes: 216 p below 2^31): the
-// (child slot, offset) -> (parent offset, child slot) table from LDS instead
-// of recomputed per entry, the four parent-map loads in flight together, one
-// 16-byte store; XCD-contiguous ranges of entries.  kmap 16-byte aligned.
-__global__ void __launch_bounds__(kThreads)
-child_kmap4_kernel(const int32_t *__restrict__ parent_kmap, int32_t p, int32_t *__restrict__ kmap) {
-    __shared__ uint8_t adj[8 * 27];  // parent offset | child slot << 5
-    if (threadIdx.x < 8 * 27) {
-        int po, cs;
-        adjacent(static_cast<int>(threadIdx.x) / 27, static_cast<int>(threadIdx.x) % 27, &po, &cs);
-        adj[threadIdx.x] = static_cast<uint8_t>(po | cs << 5);
-    }
-    __syncthreads();
-    const int32_t u = xcd_tile(blockIdx.x, gridDim.x) * kThreads + threadIdx.x;
-    const int32_t count = p * 8 * 27;
-    if (int64_t(4) * u >= count) return;
-    const int32_t g = 4 * u;
-    int32_t r = g / 27, o = g - r * 27;
-    int32_t e[4];
+// The children's rows and map in one grid: a block holds kMapPasses times eight
+// parents; thread (parent of the eight, quad) writes the same four of a parent's
+// 216 entries in every pass, so it forms their parent offsets and child slots
+// once, the passes' map loads are in flight together, and each pass's stores are
+// one contiguous 6.9 KB.  Store-bound: 195 MB of map at 226,120 parents.  (Four
+// entries a thread anywhere in the map, their places divided out per entry and
+// looked up in an LDS table, took 53.8 us and the rows' own launch 6.9; here
+// both take 40.1, 5.6 TB/s of stores.)  XCD-contiguous ranges of parents; kmap 16-byte
+// aligned (a parent's 864 bytes keep it so).
+constexpr int kMapParents = 8, kMapPasses = 4, kMapThreads = kMapParents * 54;
+__global__ void __launch_bounds__(kMapThreads)
+child_map_kernel(const int4 *__restrict__ parents, const int32_t *__restrict__ parent_kmap, int32_t p,
+                 int4 *__restrict__ children, int32_t *__restrict__ kmap) {
+    const int32_t base = xcd_tile(blockIdx.x, gridDim.x) * (kMapParents * kMapPasses);
+    const int32_t tid = threadIdx.x, own = tid / 54, quad = tid - own * 54;
+    int po[4], cs[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        e[k] = -1;
-        if (g + k < count) {
-            const uint32_t a = adj[(r & 7) * 27 + o];
-            const int32_t t = parent_kmap[(r >> 3) * 27 + static_cast<int32_t>(a & 31u)];
-            e[k] = t >= 0 ? t * 8 + static_cast<int32_t>(a >> 5) : -1;
-        }
-        if (++o == 27) o = 0, ++r;
-    }
-    if (g + 3 < count) {
-        *reinterpret_cast<int4 *>(kmap + g) = make_int4(e[0], e[1], e[2], e[3]);
-    } else {
+    for (int k = 0; k < 4; ++k) adjacent((quad * 4 + k) / 27, (quad * 4 + k) % 27, &po[k], &cs[k]);
+    int32_t t[kMapPasses][4];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (g + k < count) kmap[g + k] = e[k];
+    for (int j = 0; j < kMapPasses; ++j) {
+        const int64_t q = min(base + j * kMapParents + own, p - 1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[j][k] = parent_kmap[q * 27 + po[k]];
+    }
+    if (tid < kMapParents * kMapPasses * 8) {
+        const int32_t q = base + (tid >> 3);
+        if (q < p) children[static_cast<int64_t>(q) * 8 + (tid & 7)] = child_row(parents[q], tid & 7);
+    }
+#pragma unroll
+    for (int j = 0; j < kMapPasses; ++j) {
+        const int32_t q = base + j * kMapParents + own;
+        if (q >= p) break;
+        int32_t e[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[k] = t[j][k] >= 0 ? t[j][k] * 8 + cs[k] : -1;
+        *reinterpret_cast<int4 *>(kmap + static_cast<int64_t>(q) * 216 + quad * 4) = make_int4(e[0], e[1], e[2], e[3]);
     }
 }
 
@@ -423,16 +423,21 @@ S3DX_API s3dx_status s3dx_subdivide2(const int32_t *parent_coords, int64_t paren
         SubdivideLayout l;
         subdivide_layout(w, parent_count, &l);
         run_kmap(reinterpret_cast<const int4 *>(parent_coords), p, -1, l.parent_kmap, l.hash, s);
-        child_coords_kernel<<<blocks_for(static_cast<int64_t>(p) * 8), kThreads, 0, s>>>(
-            reinterpret_cast<const int4 *>(parent_coords), p, reinterpret_cast<int4 *>(child_coords));
-        launch_check("child_coords");
-        if (child_kmap) {
-            const int64_t entries = static_cast<int64_t>(p) * 8 * 27;
-            if (aligned(child_kmap, 16) && entries < (int64_t(1) << 31) - 4)
-                child_kmap4_kernel<<<blocks_for((entries + 3) / 4), kThreads, 0, s>>>(l.parent_kmap, p, child_kmap);
-            else
+        const int4 *parents = reinterpret_cast<const int4 *>(parent_coords);
+        int4 *children = reinterpret_cast<int4 *>(child_coords);
+        if (child_kmap && aligned(child_kmap, 16)) {
+            constexpr int kBlockParents = kMapParents * kMapPasses;
+            child_map_kernel<<<(p + kBlockParents - 1) / kBlockParents, kMapThreads, 0, s>>>(parents, l.parent_kmap, p,
+                                                                                             children, child_kmap);
+            launch_check("child_map");
+        } else {
+            child_coords_kernel<<<blocks_for(static_cast<int64_t>(p) * 8), kThreads, 0, s>>>(parents, p, children);
+            launch_check("child_coords");
+            if (child_kmap) {
+                const int64_t entries = static_cast<int64_t>(p) * 8 * 27;
                 child_kmap_kernel<<<blocks_for(entries), kThreads, 0, s>>>(l.parent_kmap, p, child_kmap);
-            launch_check("child_kmap");
+                launch_check("child_kmap");
+            }
         }
         int32_t flags[2] = {0, 0};
         hip_check(hipMemcpyAsync(flags, l.hash.flags, sizeof(flags), hipMemcpyDeviceToHost, s),
