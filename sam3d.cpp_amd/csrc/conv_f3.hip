@@ -176,6 +176,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
 #pragma unroll
             for (int i = 0; i < XP; ++i) {
                 const int sl = 64 * i + (tid >> 3);
+                // (24 bits: rows of at least 128 bytes, x below 2 GiB)
                 const uint32_t off = (__umul24(slot_row[min(sl, kF3Rows - 1)], 4u * static_cast<uint32_t>(a.cin)) +
                                       (tid & 7) * 16u) |
                                      (sl < distinct ? 0u : 0x80000000u);  // past the rows: zeros

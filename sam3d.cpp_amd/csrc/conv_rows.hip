@@ -210,9 +210,11 @@ __global__ void __launch_bounds__(256, 1) conv_rows_kernel(ConvArgs a) {
                 r_rsrc, (__attribute__((address_space(3))) void *)(smem + kRowsCap * 64 + i * 1024), 16, lane * 16,
                 kRowsTable + i * 1024, 0, 0);
     }
+    // (a full 32-bit product: at Cin 32, 64 bytes a row, x below 2 GiB holds
+    // rows above 2^24)
 #pragma unroll
     for (int i = 0; i < XP; ++i)
-        xoff[i] = (__umul24(xoff[i], 2u * static_cast<uint32_t>(a.cin)) + (tid & 3) * 16u) |
+        xoff[i] = (xoff[i] * (2u * static_cast<uint32_t>(a.cin)) + (tid & 3) * 16u) |
                   (64 * i + (tid >> 2) < distinct ? 0u : 0x80000000u);
     u32x4 xq[XP];
     auto load_x = [&](int i, int c) __attribute__((always_inline)) {

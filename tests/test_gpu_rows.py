@@ -58,3 +58,23 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
         ref = O.conv(a, m[rows], n, W.round_bf16(w), 1, cout, b)
         ref = O.silu(ref) if silu else ref
         check_rel(g[rows], ref + (res[rows >> 3] if residual else 0.0), 1e-2, "oracle")
+
+
+def test_source_rows_above_2_24(s3dx, O, W, monkeypatch):
+    # Cin 32: rows of 64 bytes, so that x below 2 GiB holds more than 2^24 rows.
+    cin, cout, n_in, n = 32, 96, (1 << 24) + 40960, 512 * 512
+    far = n_in - 40960  # every row that the map names; the rows 2^24 below are zeros
+    rng = np.random.default_rng(3)
+    x = np.zeros((n_in, cin), np.uint16)
+    x[far:] = W.f32_to_bf16_bits(rng.standard_normal((40960, cin), np.float32)).reshape(-1, cin)
+    kmap = (far + (np.arange(n)[:, None] // 64 * 5 + 31 * np.arange(27)) % 40960).astype(np.int32)
+    w, b = W.conv_weight(120, 1, cin, cout, layout="mesh"), W.normal_f32(120, 2, (cout,), 0.1)
+    one, none = s3dx.DeviceArray.from_host(np.ones(cin, np.float32)), s3dx.DeviceArray.from_host(np.zeros(cin, np.float32))
+    conv = s3dx.SparseConv(cin, cout, 27, s3dx.BF16).set_weights(w, s3dx.WEIGHT_MESH, b).set_input_affine_silu(one, none)
+    xd, kd, y = s3dx.DeviceArray.from_host(x), s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray((n, cout), np.uint16)
+    print("rows above 2^24", flush=True)
+    conv.run(xd, n_in, kd, n, y, s3dx.BF16)
+    rows = np.sort(rng.choice(n, 500, replace=False))
+    a = W.round_bf16(O.silu(W.bf16_bits_to_f32(x[far:]).reshape(-1, cin)))
+    ref = O.conv(a, kmap[rows] - far, 40960, W.round_bf16(w), 1, cout, b)
+    check_rel(W.bf16_bits_to_f32(y.download()[rows]).reshape(-1, cout), ref, 1e-2, "oracle")
