@@ -246,7 +246,9 @@ S3DX_API s3dx_status s3dx_downsample_coords(const int32_t *coords, int64_t n, in
  * records of the map at hand (a gather plan made for an FP32 layer, or input
  * transforms, whose layers make their own), BF16 MFMA on three BF16 terms of
  * every value, with no larger error against float64; bfloat16 inputs use BF16
- * MFMA; all accumulate in float32.  Deterministic (no atomics on outputs).
+ * MFMA (layers that gather parent rows behind an input affine may multiply sums
+ * of the weights that reach one parent, to 2^-27 of each sum); all accumulate in
+ * float32.  Deterministic (no atomics on outputs).
  * ---------------------------------------------------------------------- */
 typedef struct s3dx_conv s3dx_conv;
 

@@ -8,11 +8,13 @@
 // parent hold the same feature row, so
 //     sum over 27 offsets of W_o x[parent(child + o)]
 //   = sum over 8 parents of (sum of the W_o that reach it) x[parent],
-// with one set of eight folded matrices per child slot.  The folded sums
-// of the layer's BF16 weights keep two BF16 terms (a matrix that one
-// offset alone reaches is exact in one), 2^-18 of the weight, so that
-// the folding adds no error beside the BF16 rounding of the output: 15
-// matrix products per child in place of 27.
+// with one set of eight folded matrices per child slot.  A matrix that one
+// offset alone reaches is that offset's; where two reach it both are
+// multiplied as they are (two products either way); sums of four and eight are
+// held as three BF16 terms, 2^-27 of the sum, below the rounding of the FP32
+// accumulation that every kernel here has: 19 matrix products per child in
+// place of 27.  (Two terms, and 15 products, would lose what lies 2^-18 below
+// a sum.)
 //
 // Output rows 8p .. 8p + 7 of one parent are one row of 8 * cout columns, so
 // the product is a conv over the PARENTS' map whose column groups (one per
@@ -39,18 +41,31 @@ namespace {
 // on the child's side (one offset).
 constexpr int kFoldSlots = 8;
 constexpr int kFoldGroups = 8;
-// Weight steps of one (slot, 64-channel chunk): group 0 (one offset) has one
-// term, the others two; four k-steps each.
-constexpr int kFoldSteps = 4 * (1 + 2 * (kFoldGroups - 1));  // 60
+// Weight products of a group, per k-step: 1, 2, 3 or 3 for 1, 2, 4 or 8 offsets.
+__host__ __device__ constexpr int fold_terms(int m) {
+    const int axes = (m & 1) + ((m >> 1) & 1) + (m >> 2);
+    return axes < 3 ? axes + 1 : 3;
+}
+// Weight steps of one (slot, 64-channel chunk): by group, k-step (four), term.
 __host__ __device__ constexpr int fold_step(int m, int k, int term) {
-    return m == 0 ? k : 4 + ((m - 1) * 4 + k) * 2 + term;
+    int at = 0;
+    for (int g = 0; g < m; ++g) at += 4 * fold_terms(g);
+    return at + k * fold_terms(m) + term;
+}
+constexpr int kFoldSteps = fold_step(kFoldGroups - 1, 3, 2) + 1;  // 76
+static_assert(kFoldSteps == 76, "1 + 3 * 2 + 4 * 3 products a k-step");
+// The group that step t belongs to.
+constexpr int fold_group(int t) {
+    int m = 0;
+    while (t >= fold_step(m + 1, 0, 0)) ++m;
+    return m;
 }
 
 // ---------------------------------------------------------------------------
 // Folded weights from the layer's packed ones ([offset][k-step][column
 // block][lane][8]): [chunk][slot][step][column block][lane][8], the order
-// conv_fold_kernel reads them in.  One thread per 16-byte fragment pair; a
-// sum that overflows raises *bad.
+// conv_fold_kernel reads them in.  One thread per (slot, group, k-step, block,
+// lane); a weight or sum that is no finite number raises *bad.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) fold_weights_kernel(const uint4 *w, uint4 *out, int ksteps, int nbtot,
                                                            uint32_t *bad_out) {
@@ -63,7 +78,11 @@ __global__ void __launch_bounds__(256) fold_weights_kernel(const uint4 *w, uint4
         r /= nbtot;
         const int k = static_cast<int>(r & 3), m = static_cast<int>((r >> 2) & 7), s = static_cast<int>((r >> 5) & 7);
         const int c = static_cast<int>(r >> 8);
-        float sum[8] = {};
+        const int terms = fold_terms(m);
+        uint4 *dst = out + (static_cast<int64_t>(c) * kFoldSlots + s) * kFoldSteps * nbtot * 64;
+        double sum[8] = {};  // (exact: eight values of eight bits, unless 42 binary places apart)
+        bool bad = false;
+        int seen = 0;
         for (int dx = -1; dx <= 1; ++dx)
             for (int dy = -1; dy <= 1; ++dy)
                 for (int dz = -1; dz <= 1; ++dz) {
@@ -76,28 +95,30 @@ __global__ void __launch_bounds__(256) fold_weights_kernel(const uint4 *w, uint4
                     const uint32_t q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        sum[2 * e] += bf16_to_f32(static_cast<uint16_t>(q[e] & 0xffffu));
-                        sum[2 * e + 1] += bf16_to_f32(static_cast<uint16_t>(q[e] >> 16));
+                        bad = bad || (q[e] & 0x7f80u) == 0x7f80u || (q[e] & 0x7f800000u) == 0x7f800000u;
+                        sum[2 * e] += static_cast<double>(bf16_to_f32(static_cast<uint16_t>(q[e] & 0xffffu)));
+                        sum[2 * e + 1] += static_cast<double>(bf16_to_f32(static_cast<uint16_t>(q[e] >> 16)));
                     }
+                    if (terms < 3) dst[(fold_step(m, k, seen++) * nbtot + nb) * 64 + lane] = v;
                 }
-        uint32_t hi[4], lo[4];
-        bool bad = false;
+        if (terms == 3) {
+            uint32_t t[4][3];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            hi[e] = pack_bf16x2(sum[2 * e], sum[2 * e + 1]);
-            const float h0 = bf16_to_f32(static_cast<uint16_t>(hi[e] & 0xffffu)),
-                        h1 = bf16_to_f32(static_cast<uint16_t>(hi[e] >> 16));
-            bad = bad || !(__builtin_fabsf(h0) < __builtin_inff()) || !(__builtin_fabsf(h1) < __builtin_inff());
-            lo[e] = pack_bf16x2(sum[2 * e] - h0, sum[2 * e + 1] - h1);
+            for (int e = 0; e < 4; ++e) {
+                double u = sum[2 * e], v = sum[2 * e + 1];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    t[e][j] = pack_bf16x2(static_cast<float>(u), static_cast<float>(v));
+                    u -= static_cast<double>(bf16_to_f32(static_cast<uint16_t>(t[e][j] & 0xffffu)));
+                    v -= static_cast<double>(bf16_to_f32(static_cast<uint16_t>(t[e][j] >> 16)));
+                }
+                bad = bad || (t[e][0] & 0x7f80u) == 0x7f80u || (t[e][0] & 0x7f800000u) == 0x7f800000u;
+            }
+#pragma unroll
+            for (int j = 0; j < 3; ++j)  // the smallest first
+                dst[(fold_step(m, k, 2 - j) * nbtot + nb) * 64 + lane] = make_uint4(t[0][j], t[1][j], t[2][j], t[3][j]);
         }
         if (bad) *bad_out = 1u;
-        uint4 *dst = out + (static_cast<int64_t>(c) * kFoldSlots + s) * kFoldSteps * nbtot * 64;
-        if (m == 0) {
-            dst[(fold_step(0, k, 0) * nbtot + nb) * 64 + lane] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        } else {
-            dst[(fold_step(m, k, 0) * nbtot + nb) * 64 + lane] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            dst[(fold_step(m, k, 1) * nbtot + nb) * 64 + lane] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        }
     }
 }
 
@@ -196,20 +217,20 @@ __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const i
 //
 // LDS holds the parent record and two 64-channel chunks of the tile's
 // distinct rows (the next chunk's copy is spread over the current one's
-// steps).  Per (group, k-step) the four A fragments are read once for both
-// weight terms; weight fragments come straight from memory, RB steps ahead.
+// steps).  Per (group, k-step) the four A fragments are read once for all its
+// weight products; weight fragments come straight from memory, RB steps ahead.
 //
 // What bounds it: the matrix units' sustained rate.  768 -> 192 on 28,265
-// parents is 1.0 TFLOP in 742-800 us (1.25-1.35 PFLOP/s; a large BF16 matrix
-// product reaches 1.26 on this card), 192 -> 96 on 226,120 parents the same in
-// 750 us, and moving the copies, the order of the products or the waves'
-// priorities changes neither.  The 27-offset kernel took 1,491-1,553 and
-// 1,700-1,780 us.
+// parents is 1.27 TFLOP of products in 876-929 us with the row pass and the
+// plan (1.4 PFLOP/s; a large BF16 matrix product reaches 1.26 on this card), 192
+// -> 96 on 226,120 parents the same in 1,005, and moving the copies, the order
+// of the products or the waves' priorities changes neither.  The 27-offset
+// kernel takes 1,499-1,538 and 1,718 us.
 // ---------------------------------------------------------------------------
 template <int NBW>
 __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a) {
     constexpr int ROWS = 128;
-    constexpr int RB = NBW == 3 ? 2 : NBW == 2 ? 4 : 6;  // weight sets in flight
+    constexpr int RB = NBW == 3 ? 2 : 4;  // weight sets in flight
     __shared__ __align__(16) char smem[kH8Bytes];
     char *halo = smem;
     char *rec = smem + kH8Dump + 1024;
@@ -330,9 +351,9 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
         static_for<0, kFoldSteps>([&](auto tc) __attribute__((always_inline)) {
             constexpr int t = decltype(tc)::value;
             // step t: group m, k-step k, weight term
-            constexpr int m = t < 4 ? 0 : 1 + (t - 4) / 8;
-            constexpr int k = t < 4 ? t : (t - 4) / 2 % 4;
-            constexpr bool last_term = t < 4 || (t - 4) % 2 == 1;
+            constexpr int m = fold_group(t), terms = fold_terms(m);
+            constexpr int k = (t - fold_step(m, 0, 0)) / terms;
+            constexpr bool last_term = t == fold_step(m, k, terms - 1);
             constexpr bool more = t + 1 < kFoldSteps;
             // the next group's rows, once this group's last fragments are read
             if constexpr (last_term && k == 3 && more) load_ix(std::integral_constant<int, m + 1 < 8 ? m + 1 : 0>{});
@@ -355,7 +376,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
                 if constexpr (nb == NBW - 1 && last_term && more) load_a(h + 1, k == 3 ? 0 : k + 1);
                 sched_fence();
             });
-            wb = opaque_scalar<true>(wb + step_bytes);  // (a running sum: no table of 60 steps)
+            wb = opaque_scalar<true>(wb + step_bytes);  // (a running sum: no table of 76 steps)
         });
     };
     static_assert(kFoldSteps % RB == 0, "a chunk leaves every weight set at its place");
@@ -415,24 +436,26 @@ int64_t fold_weight_bytes(int cin, int blocks) {
 
 // Column blocks per workgroup of the folded conv, or 0 where the general
 // kernel suits the size.  Both sides by what they take per 64-channel chunk, in
-// microseconds: a pass of folded workgroups (one per CU) 9 per column block
+// microseconds: a pass of folded workgroups (one per CU) 11.4 per column block
 // and 18 for the plan and a tile's ends; the general kernel's 64-row tiles
-// 5.2 (96 columns) with one per CU, 9.8 with two.  Measured, folded against
-// general: 768 -> 192 on 2,000 parents 127 / 129 us, 3,000 137 / 191, 28,265
-// 800 / 1,524; 192 -> 96 on 4,000 parents 47 / 41, 8,000 53 / 76, 226,120
-// 890 / 1,710.  (Column blocks: fewer per workgroup where that fills the CUs;
-// a pass costs the same per block.)
+// 5.2 (96 columns) with one per CU, 9.8 with two, and 11.  Measured, folded against
+// general: 768 -> 192 on 2,000 parents 157 / 126 us, 3,000 152-168 / 176-187,
+// 28,265 876-929 / 1,499-1,538; 192 -> 96 on 4,800 parents 56 / 55, 6,000 58 /
+// 60, 7,200 60 / 71, 226,120 1,005 / 1,718.  Column blocks: fewer per workgroup where that
+// fills the CUs; a pass costs about the same per block (768 -> 192 on 16,000
+// parents: three blocks, one pass, 496; two blocks, two passes, 558; one
+// block, three passes, 526.  On 20,000: 813, 625 and 669).
 int fold_blocks(int cin, int blocks, int general_nb, int64_t n_parents, int64_t cus) {
     const int chunks = cin / kHChunk;
     const int64_t wgs = (n_parents + 7) / 8 * (blocks / general_nb);
     double least = chunks * general_nb / 3.0 *
-                       (wgs <= cus ? 5.2 : 9.8 * static_cast<double>(wgs) / (2.0 * static_cast<double>(cus))) + 8.0;
+                       (wgs <= cus ? 5.2 : 9.8 * static_cast<double>(wgs) / (2.0 * static_cast<double>(cus))) + 11.0;
     int best = 0;
     const int64_t tiles = (n_parents + 127) / 128;
     for (int nbw : {3, 2, 1}) {
         if (blocks % nbw != 0) continue;
         const int64_t passes = (tiles * (blocks / nbw) + cus - 1) / cus;
-        const double t = 18.0 + 9.0 * static_cast<double>(passes * nbw * chunks);
+        const double t = 18.0 + 11.4 * static_cast<double>(passes * nbw * chunks);
         if (t < least) {
             best = nbw;
             least = t;
