@@ -241,7 +241,10 @@ S3DX_API s3dx_status s3dx_downsample_coords(const int32_t *coords, int64_t n, in
  * All of it in float32, rounded once to y's dtype.  When the output tile
  * cannot span the row (Cout above 256, or not whole 32-column blocks) the
  * LayerNorm runs as a second pass over the conv's float32 output, kept in
- * another buffer the layer owns (n_out * Cout * 4 bytes, same rules).
+ * another buffer the layer owns (n_out * Cout * 4 bytes, same rules).  Layers with
+ * an input affine may also keep records of the run's map (up to 144 bytes per row of
+ * it, and a quarter more once it has grown; same rules); a run under stream capture
+ * that finds no room for them takes a kernel that needs none.
  * Arithmetic: float32 inputs use FP32 MFMA/VALU, or, in 3x3x3 layers with
  * records of the map at hand (a gather plan made for an FP32 layer, or input
  * transforms, whose layers make their own), BF16 MFMA on three BF16 terms of
@@ -257,7 +260,13 @@ S3DX_API s3dx_status s3dx_conv_create(int32_t cin, int32_t cout, int32_t kvol, i
                                       s3dx_conv **out, char *error, uint64_t error_capacity);
 S3DX_API void s3dx_conv_free(s3dx_conv *conv);
 /* host float32 weights in `layout` and optional host bias [cout]; packed once
- * into the device layout the kernel reads. */
+ * into the device layout the kernel reads.  FP32 3x3x3 layers keep their weights'
+ * three BF16 terms beside them (1.5 times the packed bytes).  3x3x3 layers that
+ * gather parent rows behind an input affine keep the sums of the weights that
+ * reach one parent (5.6 times the packed bytes for BF16, 3.6 for FP32), made when
+ * their set-up is complete: in this call, or in the s3dx_conv_set_gather_parent,
+ * _set_input_affine_silu or _set_layernorm that follows it.  Without room for
+ * either a layer runs its other kernels. */
 S3DX_API s3dx_status s3dx_conv_set_weights(s3dx_conv *conv, const float *host_weight,
                                            int32_t layout, const float *host_bias,
                                            char *error, uint64_t error_capacity);

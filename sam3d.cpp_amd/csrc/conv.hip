@@ -311,12 +311,13 @@ struct s3dx_conv {
     // that are part of a tile, grown on demand like xin.
     mutable void *sk_part = nullptr;
     mutable int64_t sk_part_bytes = 0;
-    // Folded runs (conv_fold.hip): the folded weights, their flag behind them,
-    // made in the first such run after set_weights; the state words and the
-    // parent map's records, made in every run.  Like xin, which every such
+    // Folded runs (conv_fold.hip): the folded weights, made where the layer is
+    // set up (prepare_fold; nullptr for layers that never fold, without room,
+    // and when a weight is no finite number); the state words and the parent
+    // map's records, made in every run.  The latter like xin, which every such
     // layer has.
-    mutable void *w_fold = nullptr;
-    mutable bool w_fold_ready = false;
+    void *w_fold = nullptr;
+    bool w_fold_tried = false;  // since set_weights
     mutable void *fold = nullptr;
     mutable int64_t fold_bytes = 0;
 
@@ -851,6 +852,22 @@ int gather_plan_rows(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
     return tiles <= device_cus() || stream_k_runs(conv->cin, n_out, p.grid.y) ? 128 : 64;
 }
 
+// Bytes of the layer's folded weights, 0 where none of its runs can be folded:
+// a 3x3x3 layer that gathers parent rows behind an affine, in whole 64-channel
+// chunks and column blocks (BF16) or as three BF16 terms (FP32), and below 2 GiB
+// in that form.
+int64_t fold_bytes_of(const s3dx_conv *conv) {
+    if (!conv->mfma || conv->kvol != kMaxKvol || !conv->gather_parent || conv->slot_offset || !conv->pre_scale || conv->ln ||
+        conv->cout % 32 != 0)
+        return 0;
+    int64_t bytes = 0;
+    if (conv->dtype == S3DX_F32)
+        bytes = f3_shape(conv) && (conv->w3 || !conv->weights_set) ? f3_fold_weight_bytes(conv->cin, conv->cout_pad) : 0;
+    else if (conv->cin % 64 == 0)
+        bytes = fold_weight_bytes(conv->cin, conv->cout_pad / 32);
+    return bytes < (int64_t(1) << 31) ? bytes : 0;
+}
+
 // Column blocks per workgroup of a run of folded parent rows, 0 for the
 // general kernel: a layer that reads repeated parent rows through an affine +
 // SiLU pass (so it has buffers of its own, see s3dx_conv_run) and writes rows
@@ -861,21 +878,19 @@ int gather_plan_rows(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
 int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_in, int64_t n_out,
                    bool residual, int32_t y_dtype) {
     if (!p.mfma || p.linear || !p.tl || p.xf || conv->kvol != kMaxKvol || src.shift != 3 || !conv->pre_scale ||
-        conv->ln || residual || y_dtype != conv->dtype || n_out != 8 * n_in || conv->cout % 32 != 0 ||
-        !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING") || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
+        conv->ln || residual || y_dtype != conv->dtype || n_out != 8 * n_in || !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING") || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
         (n_in + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31))
         return 0;
+    if (!fold_bytes_of(conv) || (!conv->w_fold && conv->weights_set)) return 0;
     const int blocks = conv->cout_pad / 32;
     if (conv->dtype == S3DX_F32) {
-        if (!f3_shape(conv) || !conv->w3 || f3_fold_weight_bytes(conv->cin, conv->cout_pad) >= (int64_t(1) << 31))
-            return 0;
         // In microseconds, as in f3_blocks: 64 parents' 8 slots of 32 columns a
         // workgroup, 7 per chunk.
         const int64_t passes = ((n_in + 127) / 128 * 2 * blocks + device_cus() - 1) / device_cus();
         const double fold = 25.0 + static_cast<double>(passes) * (8.0 + 7.0 * (conv->cin / 32));
         return fold < 4.0 + 54.0 * static_cast<double>(n_out) * conv->cin * conv->cout_pad / 95e6 ? 1 : 0;
     }
-    if (p.tl->id != 21 || p.half_chunk || fold_weight_bytes(conv->cin, blocks) >= (int64_t(1) << 31)) return 0;
+    if (p.tl->id != 21 || p.half_chunk) return 0;
     return fold_blocks(conv->cin, blocks, p.nb, n_in, device_cus());
 }
 
@@ -923,12 +938,71 @@ void *layer_buffer(void *&buf, int64_t &have, int64_t bytes, hipStream_t s) {
 }
 
 // The layer's buffer for what a run makes of its map: the fold state's words,
-// zeroed when the buffer is new, then `bytes` from the first KiB on.
+// zeroed when the buffer is new, then `bytes` from the first KiB on.  It grows by
+// a quarter more than asked, so that sets that grow little by little do not
+// reallocate each time.  nullptr without room, and when it would have to grow
+// while the stream is being captured (no allocation may happen then): the caller's
+// other kernel needs no such buffer.
 char *map_buffer(const s3dx_conv *conv, int64_t bytes, hipStream_t s) {
-    const int64_t had = conv->fold_bytes;
-    layer_buffer(conv->fold, conv->fold_bytes, 1024 + bytes, s);
-    if (conv->fold_bytes != had) fill_u32(static_cast<uint32_t *>(conv->fold), kFoldList, 0u, s);
+    const int64_t had = conv->fold_bytes, want = 1024 + bytes;
+    if (want > had) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone) return nullptr;
+        try {
+            layer_buffer(conv->fold, conv->fold_bytes, had ? want + want / 4 : want, s);
+        } catch (const oom_error &) {
+            (void)hipGetLastError();
+        }
+        if (!conv->fold) {
+            try {
+                layer_buffer(conv->fold, conv->fold_bytes, want, s);
+            } catch (const oom_error &) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+        }
+        fill_u32(static_cast<uint32_t *>(conv->fold), kFoldList, 0u, s);
+    }
     return static_cast<char *>(conv->fold) + 1024;
+}
+
+// Folds the weights of a layer whose runs may use them, once per set_weights, when
+// the layer's set-up is complete: by then no run has to, whatever stream it is
+// enqueued on and whether or not it is being captured.  Without room, or with
+// weights that have no finite sums, its runs take the general kernel.
+void prepare_fold(s3dx_conv *conv) {
+    const int64_t bytes = fold_bytes_of(conv);
+    if (!bytes || !conv->weights_set || conv->w_fold_tried) return;
+    conv->w_fold_tried = true;
+    // (another thread's or stream's capture has no part in this: its mode lets
+    // the calls below pass)
+    struct Relaxed {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    } relaxed;
+    struct Scratch {
+        void *d = nullptr;
+        hipStream_t s = nullptr;
+        ~Scratch() {
+            if (s) (void)hipStreamDestroy(s);
+            if (d) (void)hipFree(d);
+        }
+    } t;
+    if (hipMalloc(&t.d, static_cast<size_t>(bytes) + 16) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    hip_check(hipStreamCreateWithFlags(&t.s, hipStreamNonBlocking), "hipStreamCreate");
+    uint32_t *bad = reinterpret_cast<uint32_t *>(static_cast<char *>(t.d) + bytes), none = 1;
+    fill_u32(bad, 1, 0u, t.s);
+    if (conv->dtype == S3DX_BF16) launch_fold_weights(conv->w, t.d, conv->cin, conv->cout_pad / 32, bad, t.s);
+    else launch_f3_fold_weights(conv->w, t.d, conv->cin, conv->cout_pad, bad, t.s);
+    launch_check("fold_weights");
+    hip_check(hipMemcpyAsync(&none, bad, 4, hipMemcpyDeviceToHost, t.s), "hipMemcpyAsync folded weights");
+    hip_check(hipStreamSynchronize(t.s), "hipStreamSynchronize");
+    if (none == 0) std::swap(conv->w_fold, t.d);
 }
 
 // The layer's transformed-input buffer.
@@ -1052,7 +1126,9 @@ S3DX_API s3dx_status s3dx_conv_set_weights(s3dx_conv *conv, const float *host_we
         }
         if (conv->w) (void)hipFree(conv->w);
         conv->w = d;
-        conv->w_fold_ready = false;
+        if (conv->w_fold) (void)hipFree(conv->w_fold);
+        conv->w_fold = nullptr;
+        conv->w_fold_tried = false;
         if (conv->w_split) (void)hipFree(conv->w_split);
         conv->w_split = nullptr;
         const int nbtot = conv->cout_pad / 32;
@@ -1110,6 +1186,7 @@ S3DX_API s3dx_status s3dx_conv_set_weights(s3dx_conv *conv, const float *host_we
         }
         replace(conv->bias, upload_f32(host_bias, static_cast<size_t>(cout)));
         conv->weights_set = true;
+        prepare_fold(conv);
     });
 }
 
@@ -1121,6 +1198,7 @@ S3DX_API s3dx_status s3dx_conv_set_gather_parent(s3dx_conv *conv, int32_t enable
         conv->gather_parent = enable != 0;
         replace(conv->slot_offset,
                 enable ? upload_f32(host_slot_offset, static_cast<size_t>(8) * conv->cin) : nullptr);
+        prepare_fold(conv);
     });
 }
 
@@ -1132,6 +1210,7 @@ S3DX_API s3dx_status s3dx_conv_set_input_affine_silu(s3dx_conv *conv, const floa
         require((scale == nullptr) == (shift == nullptr), "scale and shift must both be set");
         conv->pre_scale = scale;
         conv->pre_shift = shift;
+        prepare_fold(conv);
     });
 }
 
@@ -1153,6 +1232,7 @@ S3DX_API s3dx_status s3dx_conv_set_layernorm(s3dx_conv *conv, int32_t enable, fl
         replace(conv->mod_scale, enable ? upload_f32(host_mod_scale, c) : nullptr);
         replace(conv->mod_shift, enable ? upload_f32(host_mod_shift, c) : nullptr);
         if (!enable) conv->dmod_scale = conv->dmod_shift = nullptr;
+        prepare_fold(conv);
     });
 }
 
@@ -1299,21 +1379,16 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         LaunchPlan plan = plan_launch(conv, x_bytes, n_out, aligned16, bf16_rows,
                                       residual == nullptr && y_dtype == S3DX_BF16);
         int fold = xvec ? fold_blocks_of(conv, plan, src, n_in, n_out, residual != nullptr, y_dtype) : 0;
-        uint32_t *fold_state = nullptr, *fold_bad = nullptr;
-        void *fold_records = nullptr;
+        uint32_t *fold_state = nullptr;
+        char *fold_records = nullptr;
         if (fold) {
             const int64_t tiles = (n_in + 127) / 128;
             const int64_t list = static_cast<int64_t>(round_up((kFoldList + tiles) * 4, 1024)) - 1024;
-            const int64_t fw = bf ? fold_weight_bytes(conv->cin, conv->cout_pad / 32)
-                                  : f3_fold_weight_bytes(conv->cin, conv->cout_pad);
-            try {
-                fold_records = map_buffer(conv, list + tiles * kGatherPlanRecord128, s) + list;
-                if (!conv->w_fold) hip_check(hipMalloc(&conv->w_fold, static_cast<size_t>(fw) + 16), "hipMalloc");
+            fold_records = map_buffer(conv, list + tiles * kGatherPlanRecord128, s);
+            if (fold_records) {
+                fold_records += list;
                 fold_state = static_cast<uint32_t *>(conv->fold);
-                fold_bad = reinterpret_cast<uint32_t *>(static_cast<char *>(conv->w_fold) + fw);
-            } catch (const oom_error &) {  // no room for the folding's buffers: the general kernel
-                (void)hipGetLastError();
-                fold_state = nullptr;
+            } else {
                 fold = 0;
             }
         }
@@ -1322,11 +1397,10 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         const int64_t row_list = static_cast<int64_t>(round_up((kFoldList + row_tiles) * 4, 1024)) - 1024;
         char *row_records = nullptr;
         if (!gplan && xvec && aligned16 && rows_of(conv, plan, src, n_out, y_dtype)) {
-            try {
-                row_records = map_buffer(conv, row_list + row_tiles * kRowsRecord, s) + row_list;
+            row_records = map_buffer(conv, row_list + row_tiles * kRowsRecord, s);
+            if (row_records) {
+                row_records += row_list;
                 fold_state = static_cast<uint32_t *>(conv->fold);
-            } catch (const oom_error &) {
-                (void)hipGetLastError();
             }
         }
         if (src.pre) {
@@ -1398,14 +1472,7 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             a.w3 = conv->w3;
         }
         if (fold) {
-            if (!conv->w_fold_ready) {
-                fill_u32(fold_bad, 1, 0u, s);
-                if (bf) launch_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad / 32, fold_bad, s);
-                else launch_f3_fold_weights(conv->w, conv->w_fold, conv->cin, conv->cout_pad, fold_bad, s);
-                launch_check("fold_weights");
-                conv->w_fold_ready = true;
-            }
-            launch_fold_plan(kmap, n_in, fold_records, fold_state, fold_bad, !bf, s);
+            launch_fold_plan(kmap, n_in, fold_records, fold_state, !bf, s);
             launch_check("fold_plan");
             ConvArgs fa = a;
             fa.plan = fold_records;
@@ -1436,14 +1503,12 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         if (!gplan && aligned16) {
             const LaunchPlan whole = plan;
             if (f3_own_plan(conv, plan, src, n_out)) {
-                try {
-                    void *records = map_buffer(conv, (n_out + 127) / 128 * kGatherPlanRecord128, s);
+                if (char *records = map_buffer(conv, (n_out + 127) / 128 * kGatherPlanRecord128, s)) {
                     launch_gather_plan_build(128, kmap, n_out, src.n_src, src.shift, records, s);
                     launch_check("gather_plan_build");
                     a.plan = records;
                     a.w3 = conv->w3;
-                } catch (const oom_error &) {
-                    (void)hipGetLastError();
+                } else {
                     plan = whole;
                 }
             }

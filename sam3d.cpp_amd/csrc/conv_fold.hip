@@ -134,8 +134,7 @@ struct FoldSlice {
 };
 
 __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const int32_t *kmap, int64_t n_parents,
-                                                                         char *plan, uint32_t *state,
-                                                                         const uint32_t *bad_weights, int most) {
+                                                                         char *plan, uint32_t *state, int most) {
     // A parent's 8 * 27 child entries are 54 16-byte pieces; 864 of the threads
     // take the pieces of 16 parents a pass, each thread the same piece of
     // every parent, so that what its four entries are (the parent offset they
@@ -175,7 +174,7 @@ __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const i
         d[k] = (px + 1) * 9 + (py + 1) * 3 + pz + 1;
         kept[k] = o == d[k] && s == ((px == 1) << 2 | (py == 1) << 1 | int(pz == 1));
     }
-    if (tid == 0) wrong = state[kFoldBadRows] | *bad_weights;
+    if (tid == 0) wrong = state[kFoldBadRows];
     int32_t pj[Q][4];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -471,11 +470,10 @@ void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t
                        bad);
 }
 
-void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
-                      bool f32, hipStream_t stream) {
+void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, bool f32, hipStream_t stream) {
     hipLaunchKernelGGL(fold_plan_kernel, dim3(static_cast<unsigned>((n_parents + 127) / 128)),
                        dim3(kPlanBuild128Threads), 0, stream, kmap, n_parents, static_cast<char *>(plan), state,
-                       bad_weights, f32 ? kF3MostRows : kH8Double);
+                       f32 ? kF3MostRows : kH8Double);
 }
 
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream) {

@@ -134,8 +134,7 @@ int64_t fold_weight_bytes(int cin, int blocks);
 int fold_blocks(int cin, int blocks, int general_nb, int64_t n_parents, int64_t cus);
 // *bad: raised when a folded weight is no finite number.
 void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t *bad, hipStream_t stream);
-void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, const uint32_t *bad_weights,
-                      bool f32, hipStream_t stream);
+void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, bool f32, hipStream_t stream);
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
 // The general kernel (64-row tiles, nb column blocks) over the listed tiles of
 // `per` * 64 rows.

@@ -9,6 +9,8 @@ one BF16 step here and there (rel-L2 far below 2^-9).  Parent tiles whose map
 is not a subdivide's, or rows that hold an infinity, go to the 27-offset
 kernel: those outputs are the same bits.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -155,3 +157,79 @@ def test_folded_sums_keep_fp32s_bits(s3dx, W, offsets):
     # (a row's own rounding to BF16 can go the other way where silu ties: 2^-8)
     print(f"offsets {offsets}: worst {err.max():.2e}, median {np.median(err):.2e}", flush=True)
     assert err.max() < 2.0 ** -3.5 + 2.0 ** -8
+
+
+class _Capture:
+    """A HIP graph of what is enqueued on a stream inside the with block."""
+
+    def __init__(self, stream):
+        with open("/proc/self/maps") as f:
+            self.hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+        self.stream, self.graph, self.exec = C.c_void_p(stream.handle), C.c_void_p(), C.c_void_p()
+
+    def __enter__(self):
+        assert self.hip.hipStreamBeginCapture(self.stream, 0) == 0
+        return self
+
+    def __exit__(self, *exc):
+        assert self.hip.hipStreamEndCapture(self.stream, C.byref(self.graph)) == 0
+        if exc[0] is None:
+            assert self.hip.hipGraphInstantiate(C.byref(self.exec), self.graph, None, None, C.c_size_t(0)) == 0
+
+    def launch(self):
+        assert self.hip.hipGraphLaunch(self.exec, self.stream) == 0
+        assert self.hip.hipStreamSynchronize(self.stream) == 0
+
+    def close(self):
+        for f, h in ((self.hip.hipGraphExecDestroy, self.exec), (self.hip.hipGraphDestroy, self.graph)):
+            if h:
+                f(h)
+
+
+def test_new_weights_then_capture(s3dx, W):
+    # The first run after set_weights is captured, and nothing has replayed it
+    # when the next run is made: neither may see the weights before.
+    p, cin, cout = 20011, 192, 96
+    conv, kmap, x, w, b, *_ = _setup(s3dx, W, W.shells_union(0)[:p], cin, cout)
+    xd, kd = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(x)), s3dx.DeviceArray.from_host(kmap)
+    ys = [s3dx.DeviceArray((8 * p, cout), np.uint16) for _ in range(2)]
+    stream = s3dx.Stream()
+
+    def run(y):
+        conv.run(xd, p, kd, 8 * p, y, s3dx.BF16, stream=stream)
+
+    run(ys[0])
+    stream.synchronize()
+    first = ys[0].download()
+    conv.set_weights(2.0 * w, s3dx.WEIGHT_MESH, 2.0 * b)  # (twice: exact in BF16)
+    print("capture after set_weights", flush=True)
+    with _Capture(stream) as graph:
+        run(ys[1])
+    for _ in range(3):
+        run(ys[0])
+        stream.synchronize()
+        assert np.array_equal(W.bf16_bits_to_f32(ys[0].download()), 2.0 * W.bf16_bits_to_f32(first))
+        ys[1].upload(np.zeros((8 * p, cout), np.uint16))
+        graph.launch()
+        assert np.array_equal(ys[1].download(), ys[0].download())
+    graph.close()
+
+
+def test_capture_with_no_room_yet(s3dx, W, monkeypatch):
+    # A layer whose runs had no map records so far: the captured run can make none
+    # and takes the 27-offset kernel; the next eager run is folded.
+    p, cin, cout = 20011, 192, 96
+    conv, kmap, x, *_ = _setup(s3dx, W, W.shells_union(0)[:p], cin, cout)
+    xd, kd, y = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(x)), s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray((8 * p, cout), np.uint16)
+    general = _general(s3dx, W, monkeypatch, conv, x, kmap, cout)
+    stream = s3dx.Stream()
+    print("capture before the first folded run", flush=True)
+    with _Capture(stream) as graph:
+        conv.run(xd, p, kd, 8 * p, y, s3dx.BF16, stream=stream)
+    folded = _run(s3dx, W, conv, x, kmap, cout)
+    for _ in range(3):
+        graph.launch()
+        assert np.array_equal(y.download(), general)
+        assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), folded)
+    graph.close()
+    assert not np.array_equal(folded, general)
