@@ -823,8 +823,8 @@ void apply_gather_plan(LaunchPlan &p, const s3dx_conv *conv, const s3dx_gather_p
     }
 }
 
-// An unplanned run of an FP32 layer that has buffers of its own (input
-// transforms): as three BF16 terms, with the map's 128-row records built in
+// A run, over no plan that it could read, of an FP32 layer that has buffers of its
+// own (input transforms): as three BF16 terms, with the map's 128-row records built in
 // the run where that pays (about 10 us).
 bool f3_own_plan(const s3dx_conv *conv, LaunchPlan &p, const Source &src, int64_t n_out) {
     if (!src.pre || conv->dtype != S3DX_F32 || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
@@ -894,7 +894,7 @@ int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src
     return fold_blocks(conv->cin, blocks, p.nb, n_in, device_cus());
 }
 
-// Whether a run goes by 512-row tiles (conv_rows.hip): an unplanned BF16 layer
+// Whether a run goes by 512-row tiles (conv_rows.hip): a BF16 layer
 // with an input affine (so with buffers of its own) that no halo kernel suits
 // (Cin 32 above a multiple of 64), 96-column groups, BF16 output and no
 // LayerNorm, over at least as many tiles as CUs (96 -> 96 on 256,000 rows: 176
@@ -907,6 +907,58 @@ bool rows_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int6
            n_out * kMaxKvol * 4 < (int64_t(1) << 31) && (n_out + 511) / 512 * int64_t(kRowsRecord) < (int64_t(1) << 31) &&
            int64_t(kMaxKvol) * conv->cin * conv->cout_pad * 2 < (int64_t(1) << 31) &&
            (n_out + 511) / 512 * (conv->cout / 96) >= device_cus();
+}
+
+// Whether the transforms run on 16-byte pieces with 32-bit piece indices (else
+// one element per thread).
+bool xvec_of(const s3dx_conv *conv, const Source &src) {
+    const int e = conv->dtype == S3DX_BF16 ? 8 : 4;
+    return conv->cin % e == 0 && src.rows * (conv->cin / e) < (int64_t(1) << 32) && aligned(conv->pre_scale, 16) &&
+           aligned(conv->pre_shift, 16);
+}
+
+// How a run is launched, decided on the host from sizes, types and alignment
+// alone; shared by s3dx_conv_run and s3dx_conv_plan.
+struct Route {
+    LaunchPlan p;          // the kernel; with fold or rows the one for the tiles they leave over
+    LaunchPlan whole;      // own: the kernel without the records
+    int fold = 0;          // folded parent rows: 32-column blocks per workgroup
+    bool rows = false;     // 512-row tiles
+    bool planned = false;  // the kernel reads the caller's gather plan
+    bool own = false;      // records of the map are built in the run (p.f3)
+    bool widen = false;    // BF16 rows are widened for an FP32 layer first
+};
+
+// aligned16: map, output and residual are 16-byte aligned.  xvec: the transforms
+// run on 16-byte pieces.
+Route route_of(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const Source &src, int64_t n_in, int64_t n_out,
+               bool aligned16, bool xvec, bool residual, int32_t y_dtype) {
+    if (gplan)
+        require(gplan->n_out == n_out && gplan->n_src == src.n_src && gplan->shift == src.shift,
+                "gather plan was built for another map size or source rows");
+    Route r;
+    const bool bf16_rows = conv->in_dtype != conv->dtype;  // BF16 rows into an FP32 layer
+    const int64_t count = src.rows * conv->cin;
+    r.p = plan_launch(conv, count * dtype_size(conv->in_dtype), n_out, aligned16, bf16_rows,
+                      !residual && y_dtype == S3DX_BF16);
+    r.widen = bf16_rows && !r.p.linear;
+    if (r.widen) r.p = plan_launch(conv, count * 4, n_out, aligned16);
+    if (xvec) {
+        r.fold = fold_blocks_of(conv, r.p, src, n_in, n_out, residual, y_dtype);
+        r.rows = !r.fold && !gplan && rows_of(conv, r.p, src, n_out, y_dtype);
+        if (r.fold || r.rows) return r;
+    }
+    if (gplan) {
+        // Only the halo kernels and the three-term one read plans; other launches ignore it.
+        apply_gather_plan(r.p, conv, gplan, n_out, bf16_rows);
+        r.planned = r.p.fn == pick_halo_bf16_planned(64) || r.p.fn == pick_halo_bf16_planned(128) ||
+                    r.p.fn == pick_halo_bf16_planned(64, 3) || r.p.f3 || (r.p.stream_k && !r.p.sk_splitk);
+    }
+    if (!r.planned) {
+        r.whole = r.p;
+        r.own = !gplan && f3_own_plan(conv, r.p, src, n_out);
+    }
+    return r;
 }
 
 float *upload_f32(const float *host, size_t count) {
@@ -1289,19 +1341,8 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
         require(conv->kvol != 1 || n_out <= src.n_src,
                 "n_out exceeds the input rows (kvol 1 without a map reads row i of x)");
         const bool bf16_rows = conv->in_dtype != conv->dtype;
-        const int64_t x_bytes = src.rows * conv->cin * static_cast<int64_t>(dtype_size(conv->in_dtype));
-        LaunchPlan p = plan_launch(conv, x_bytes, n_out, true, bf16_rows);
-        const bool widen = bf16_rows && !p.linear;
-        if (widen) p = plan_launch(conv, src.rows * conv->cin * 4, n_out, true);
-        if (!gplan) f3_own_plan(conv, p, src, n_out);
-        if (gplan) {
-            require(gplan->n_out == n_out && gplan->n_src == src.n_src && gplan->shift == src.shift,
-                    "gather plan was built for another map size or source rows");
-            apply_gather_plan(p, conv, gplan, n_out, bf16_rows);
-        }
-        const bool planned = gplan && (p.fn == pick_halo_bf16_planned(64) || p.fn == pick_halo_bf16_planned(128) ||
-                                       p.fn == pick_halo_bf16_planned(64, 3) || p.f3 ||
-                                       (p.stream_k && !p.sk_splitk));
+        const Route r = route_of(conv, gplan, src, n_in, n_out, true, xvec_of(conv, src), false, conv->dtype);
+        const LaunchPlan &p = r.p;
         char text[256];
         const bool halo = p.mfma && !p.linear && p.tl->id >= 20 && p.tl->id <= 22;  // the halo-staged kernels
         char groups[16] = "";
@@ -1321,9 +1362,19 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
         else
             std::snprintf(text, sizeof(text), "generic rows=%d cols=%d ln=%s grid=%ux%u", kGM, kGN,
                           conv->ln ? "separate" : "none", p.grid.x, p.grid.y);
-        std::snprintf(plan, plan_capacity, "%s%s%s%s%s", bf16_rows ? (widen ? "in=bf16 pre=widen " : "in=bf16 ") : "",
+        // (the kernel of most tiles, and "else" the one of those it leaves over)
+        char most[96] = "";
+        if (r.fold)
+            std::snprintf(most, sizeof(most), "fold%s rows=%d cols=%d grid=%lldx%d else ", conv->dtype == S3DX_F32 ? " terms=3" : "",
+                          conv->dtype == S3DX_F32 ? 512 : 1024, r.fold * 32,
+                          static_cast<long long>((n_in + 127) / 128 * (conv->dtype == S3DX_F32 ? 2 : 1)),
+                          conv->cout_pad / 32 / r.fold);
+        else if (r.rows)
+            std::snprintf(most, sizeof(most), "rows=512 cols=96 grid=%lldx%d else ", static_cast<long long>((n_out + 511) / 512),
+                          conv->cout / 96);
+        std::snprintf(plan, plan_capacity, "%s%s%s%s%s%s", bf16_rows ? (r.widen ? "in=bf16 pre=widen " : "in=bf16 ") : "",
                       src.pre ? (src.children ? "pre=children " : "pre=rows ") : "", src.shift ? "parent-rows " : "",
-                      text, planned ? (gplan->rows == 128 ? " plan=128" : " plan=64") : "");
+                      most, text, r.planned ? (gplan->rows == 128 ? " plan=128" : " plan=64") : r.own ? " plan=own" : "");
     }
 }
 
@@ -1372,13 +1423,10 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         const int64_t x_bytes = src.rows * conv->cin * static_cast<int64_t>(dtype_size(conv->in_dtype));
         // The MFMA kernel reads the map and writes rows with 16-byte accesses.
         const bool aligned16 = aligned(kmap, 16) && aligned(y, 16) && aligned(residual, 16);
-        // 16-byte pieces with 32-bit piece indices; else one element per thread.
-        const bool xvec = conv->cin % (bf ? 8 : 4) == 0 &&
-                          src.rows * (conv->cin / (bf ? 8 : 4)) < (int64_t(1) << 32) &&
-                          aligned(conv->pre_scale, 16) && aligned(conv->pre_shift, 16);
-        LaunchPlan plan = plan_launch(conv, x_bytes, n_out, aligned16, bf16_rows,
-                                      residual == nullptr && y_dtype == S3DX_BF16);
-        int fold = xvec ? fold_blocks_of(conv, plan, src, n_in, n_out, residual != nullptr, y_dtype) : 0;
+        const bool xvec = xvec_of(conv, src);
+        const Route route = route_of(conv, gplan, src, n_in, n_out, aligned16, xvec, residual != nullptr, y_dtype);
+        LaunchPlan plan = route.p;
+        int fold = route.fold;
         uint32_t *fold_state = nullptr;
         char *fold_records = nullptr;
         if (fold) {
@@ -1396,7 +1444,7 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         const int64_t row_tiles = (n_out + 511) / 512;
         const int64_t row_list = static_cast<int64_t>(round_up((kFoldList + row_tiles) * 4, 1024)) - 1024;
         char *row_records = nullptr;
-        if (!gplan && xvec && aligned16 && rows_of(conv, plan, src, n_out, y_dtype)) {
+        if (route.rows) {
             row_records = map_buffer(conv, row_list + row_tiles * kRowsRecord, s);
             if (row_records) {
                 row_records += row_list;
@@ -1414,10 +1462,9 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             xa.slot_offset = conv->slot_offset;
             xa.scale = conv->pre_scale;
             xa.shift = conv->pre_shift;
-            const bool vec = xvec;
-            const int64_t items = src.rows * (vec ? conv->cin / (bf ? 8 : 4) : conv->cin);
+            const int64_t items = src.rows * (xvec ? conv->cin / (bf ? 8 : 4) : conv->cin);
             const dim3 grid(static_cast<unsigned>(std::min<int64_t>((items + 255) / 256, 16384)));
-            if (vec) {
+            if (xvec) {
                 if (bf) hipLaunchKernelGGL(xform_rows_kernel<uint16_t>, grid, dim3(256), 0, s, xa);
                 else hipLaunchKernelGGL(xform_rows_kernel<float>, grid, dim3(256), 0, s, xa);
             } else {
@@ -1450,27 +1497,18 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         a.ln_b = conv->ln_b;
         a.mod_scale = conv->dmod_scale ? conv->dmod_scale : conv->mod_scale;
         a.mod_shift = conv->dmod_scale ? conv->dmod_shift : conv->mod_shift;
-        if (bf16_rows && !plan.linear) {
-            // Other kernels read the layer's dtype: the rows are widened
-            // (exactly) once, into the layer's buffer.
+        if (route.widen) {
+            // Kernels other than the 1x1 ones read the layer's dtype: the rows
+            // are widened (exactly) once, into the layer's buffer.
             const int64_t count = src.rows * conv->cin;
             void *xw = transform_buffer(conv, count * 4, s);
             convert_launch(x, S3DX_BF16, count, xw, S3DX_F32, s);
             a.x = xw;
             a.x_bytes = count * 4;
-            plan = plan_launch(conv, a.x_bytes, n_out, aligned16);
         }
         if (plan.split) a.w = conv->w_split;
-        if (gplan) {
-            require(gplan->n_out == n_out && gplan->n_src == src.n_src && gplan->shift == src.shift,
-                    "gather plan was built for another map size or source rows");
-            // Only the halo kernels read plans; other launches ignore it.
-            apply_gather_plan(plan, conv, gplan, n_out, bf16_rows);
-            if (plan.fn == pick_halo_bf16_planned(64) || plan.fn == pick_halo_bf16_planned(128) ||
-                plan.fn == pick_halo_bf16_planned(64, 3) || plan.f3 || plan.stream_k)
-                a.plan = gplan->d;
-            a.w3 = conv->w3;
-        }
+        if (route.planned) a.plan = gplan->d;
+        if (plan.f3) a.w3 = conv->w3;
         if (fold) {
             launch_fold_plan(kmap, n_in, fold_records, fold_state, !bf, s);
             launch_check("fold_plan");
@@ -1500,17 +1538,13 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             launch_check("conv_halo_listed");
             return;
         }
-        if (!gplan && aligned16) {
-            const LaunchPlan whole = plan;
-            if (f3_own_plan(conv, plan, src, n_out)) {
-                if (char *records = map_buffer(conv, (n_out + 127) / 128 * kGatherPlanRecord128, s)) {
-                    launch_gather_plan_build(128, kmap, n_out, src.n_src, src.shift, records, s);
-                    launch_check("gather_plan_build");
-                    a.plan = records;
-                    a.w3 = conv->w3;
-                } else {
-                    plan = whole;
-                }
+        if (route.own) {
+            if (char *records = map_buffer(conv, (n_out + 127) / 128 * kGatherPlanRecord128, s)) {
+                launch_gather_plan_build(128, kmap, n_out, src.n_src, src.shift, records, s);
+                launch_check("gather_plan_build");
+                a.plan = records;
+            } else {
+                plan = route.whole;
             }
         }
         // A LayerNorm the epilogue cannot fuse runs as its own pass over the

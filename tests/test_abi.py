@@ -162,6 +162,31 @@ def test_conv_plan_names_the_launched_kernel(s3dx, monkeypatch):
         c128.plan(0, n)
 
 
+def test_conv_plan_names_the_mesh_layers_kernels(s3dx, monkeypatch):
+    # The mesh decoder's convs, at sizes where each of their kernels runs (256 CUs
+    # without a device); fake addresses for the affine, which a query does not read.
+    for e in ("S3DX_CONV_TILING", "S3DX_CONV_HALO"):
+        monkeypatch.delenv(e, raising=False)
+
+    def text(cin, cout, dtype, n_in, n_out, parent):
+        conv = s3dx.SparseConv(cin, cout, 27, dtype).set_gather_parent(parent)
+        return conv.set_input_affine_silu(0x1000, 0x2000).plan(n_in, n_out)
+
+    p = 28265
+    assert text(768, 192, s3dx.BF16, p, 8 * p, True) == \
+        "pre=rows parent-rows fold rows=1024 cols=96 grid=221x2 else mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 " \
+        "ln=none grid=3534x2"
+    assert text(768, 192, s3dx.BF16, p, 8 * p - 8, True).startswith("pre=rows parent-rows mfma tiling=21 ")
+    assert text(768, 192, s3dx.BF16, 300, 2400, True).startswith("pre=rows parent-rows mfma tiling=21 ")
+    assert text(96, 96, s3dx.BF16, 64 * p, 64 * p, False) == \
+        "pre=rows rows=512 cols=96 grid=3534x1 else mfma tiling=19 split-k rows=64 cols=96 kc=32 xf=0 ln=none grid=28265x1"
+    assert text(768, 192, s3dx.F32, 6001, 8 * 6001, True).startswith("pre=rows parent-rows fold terms=3 rows=512 cols=32 grid=94x6 else ")
+    assert text(192, 192, s3dx.F32, 48008, 48008, False) == \
+        "pre=rows mfma tiling=25 terms=3 rows=128 cols=64 kc=32 xf=0 ln=none grid=376x3 plan=own"
+    monkeypatch.setenv("S3DX_CONV_TILING", "21")
+    assert text(768, 192, s3dx.BF16, p, 8 * p, True).startswith("pre=rows parent-rows mfma tiling=21 ")
+
+
 def test_missing_library_fails_loudly(s3dx, monkeypatch, tmp_path):
     monkeypatch.setattr(s3dx, "_lib", None)
     monkeypatch.setattr(s3dx, "LIB_PATH", tmp_path / "absent.so")

@@ -137,12 +137,12 @@ def _parent_map(kmap):
 # level (conv1 gathering parent rows after the GN affine + SiLU pass, the 1x1
 # skip on the parents, conv2 after its GN pass).
 CONFIG5_PLANS = {
-    0: ("pre=rows parent-rows mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 ln=none grid=3534x2",
+    0: ("pre=rows parent-rows fold rows=1024 cols=96 grid=221x2 else mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 ln=none grid=3534x2",
         "mfma tiling=4 rows=64 cols=192 kc=64 xf=0 ln=none grid=442x1",
         "pre=rows mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 ln=none grid=3534x2"),
-    1: ("pre=rows parent-rows mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 ln=none grid=28265x1",
+    1: ("pre=rows parent-rows fold rows=1024 cols=96 grid=1767x1 else mfma tiling=21 split-k halo rows=64 cols=96 kc=64 xf=0 ln=none grid=28265x1",
         "linear pipe cols=96 ksteps=12 ln=none grid=512",
-        "pre=rows mfma tiling=19 split-k rows=64 cols=96 kc=32 xf=0 ln=none grid=28265x1"),
+        "pre=rows rows=512 cols=96 grid=3534x1 else mfma tiling=19 split-k rows=64 cols=96 kc=32 xf=0 ln=none grid=28265x1"),
 }
 
 

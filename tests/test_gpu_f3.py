@@ -183,7 +183,10 @@ def _run(s3dx, conv, x, kmap, cout):
 ])
 def test_layers_with_transforms(s3dx, W, monkeypatch, p, cin, cout, parent):
     conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, parent)
-    print(f"p={p} {cin}->{cout} parent={parent}: {conv.plan(x.shape[0], 8 * p)}", flush=True)
+    text = conv.plan(x.shape[0], 8 * p)
+    print(f"p={p} {cin}->{cout} parent={parent}: {text}", flush=True)
+    assert (f" fold terms=3 rows=512 cols=32 grid={(p + 127) // 128 * 2}x{cout // 32} else " if parent else " tiling=25 terms=3 rows=128 ") in text
+    assert parent or text.endswith(" plan=own")
     got = _run(s3dx, conv, x, kmap, cout)
     assert np.array_equal(got, _run(s3dx, conv, x, kmap, cout)), "two runs differ"
     monkeypatch.setenv("S3DX_CONV_TILING", "11")
@@ -202,6 +205,7 @@ def test_folded_fp32_maps_and_infinities(s3dx, W, monkeypatch):
     # instructions: near the FP32 kernel's values, the same infinities and NaN.
     p, cin, cout = 3001, 64, 96
     conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, True)
+    assert " fold terms=3 " in conv.plan(p, 8 * p)
     bad = kmap.copy()
     bad[8 * 130 + 3, 14] = -1
     bad[8 * 300, 26] = 8 * 2000 + 1

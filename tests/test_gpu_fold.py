@@ -46,24 +46,26 @@ def _general(s3dx, W, monkeypatch, *args, **kw):
     return y
 
 
-@pytest.mark.parametrize("p,cin,cout,silu", [
-    (6007, 192, 96, False),   # one column block a workgroup; a ragged last parent tile
-    (20011, 192, 96, True),   # three
-    (12801, 64, 192, False),  # one chunk; a last tile of one parent
-    (9000, 128, 128, False),  # column blocks in twos
-    (4000, 768, 192, False),  # the mesh decoder's first level
+@pytest.mark.parametrize("p,cin,cout,silu,cols", [
+    (6007, 192, 96, False, 32),   # one column block a workgroup; a ragged last parent tile
+    (20011, 192, 96, True, 32),   # the same in two passes over the CUs
+    (24011, 192, 96, True, 96),   # three
+    (12801, 64, 192, False, 96),  # one chunk; a last tile of one parent
+    (9000, 128, 128, False, 64),  # column blocks in twos
+    (4000, 768, 192, False, 32),  # the mesh decoder's first level
 ])
-def test_folded_matches_general_and_oracle(s3dx, O, W, monkeypatch, p, cin, cout, silu):
+def test_folded_matches_general_and_oracle(s3dx, O, W, monkeypatch, p, cin, cout, silu, cols):
     parents = W.shells_union(0)[:p]
     conv, kmap, x, w, b, scale, shift = _setup(s3dx, W, parents, cin, cout, silu)
-    print(f"fold p={p} {cin}->{cout} silu={silu}", flush=True)
+    print(f"fold p={p} {cin}->{cout} silu={silu}: {conv.plan(p, 8 * p)}", flush=True)
+    assert f" fold rows=1024 cols={cols} grid={(p + 127) // 128}x{cout // cols} else mfma tiling=21 " in conv.plan(p, 8 * p)
     got = _run(s3dx, W, conv, x, kmap, cout)
     assert np.array_equal(got, _run(s3dx, W, conv, x, kmap, cout)), "two runs differ"
     want = _general(s3dx, W, monkeypatch, conv, x, kmap, cout)
     g, v = W.bf16_bits_to_f32(got).reshape(got.shape), W.bf16_bits_to_f32(want).reshape(got.shape)
     rel = float(np.linalg.norm(g - v) / np.linalg.norm(v))
     print(f"  against the 27-offset kernel: rel-L2 {rel:.2e}, same bits {np.mean(got == want):.4f}", flush=True)
-    assert 0.0 < rel < 2.0 ** -11  # (0: the folded kernel did not run)
+    assert 0.0 < rel < 2.0 ** -11
     rows = np.sort(np.random.default_rng(1).choice(8 * p, 1500, replace=False))
     rows = np.unique(np.concatenate([rows, [0, 1023, 1024, 8 * p - 1]]))
     a = W.round_bf16(O.silu((x * scale + shift).astype(np.float32)))
@@ -97,6 +99,7 @@ def test_maps_no_subdivide_made(s3dx, W, monkeypatch):
     assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout)[:1024], got[:1024])
     # fewer rows than eight per parent: the general kernel
     n = 8 * p - 8
+    assert " fold " in conv.plan(p, 8 * p) and " fold " not in conv.plan(p, n)
     assert np.array_equal(_run(s3dx, W, conv, x, kmap[:n], cout, n), _general(s3dx, W, monkeypatch, conv, x, kmap[:n], cout, n))
 
 
@@ -122,7 +125,9 @@ def test_infinities_new_weights_and_sizes(s3dx, W, monkeypatch):
     # a weight whose folded sum overflows: the 27-offset kernel
     wh = w.copy()
     wh[:, 0, 0] = 2.0e38
+    assert " fold " in conv.plan(7000, 56000)
     conv.set_weights(wh, s3dx.WEIGHT_MESH, b)
+    assert " fold " not in conv.plan(7000, 56000)
     assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), _general(s3dx, W, monkeypatch, conv, x, kmap, cout))
 
 
@@ -155,6 +160,7 @@ def test_folded_sums_keep_fp32s_bits(s3dx, W, offsets):
     at = np.flatnonzero(rows[:, 2] >= 0)
     err = np.abs(y[at, 0] - want[at]) / np.abs(want[at])
     # (a row's own rounding to BF16 can go the other way where silu ties: 2^-8)
+    assert " fold " in conv.plan(p, 8 * p)
     print(f"offsets {offsets}: worst {err.max():.2e}, median {np.median(err):.2e}", flush=True)
     assert err.max() < 2.0 ** -3.5 + 2.0 ** -8
 
@@ -233,3 +239,19 @@ def test_capture_with_no_room_yet(s3dx, W, monkeypatch):
         assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), folded)
     graph.close()
     assert not np.array_equal(folded, general)
+
+
+def test_refused_plan_leaves_nothing_behind(s3dx, W):
+    # A plan of another size is refused before anything is enqueued: rows with an
+    # infinity in that call do not send the next one to the 27-offset kernel.
+    p, cin, cout = 9000, 192, 96
+    conv, kmap, x, *_ = _setup(s3dx, W, W.shells_union(0)[:p], cin, cout)
+    first = _run(s3dx, W, conv, x, kmap, cout)
+    kd = s3dx.DeviceArray.from_host(kmap)
+    gp = conv.gather_plan(p, kd, 8 * p - 8)
+    xi = x.copy()
+    xi[500, 7] = np.inf
+    y = s3dx.DeviceArray((8 * p, cout), np.uint16)
+    with pytest.raises(s3dx.S3dxError):
+        conv.run(s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(xi)), p, kd, 8 * p, y, s3dx.BF16, plan=gp)
+    assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), first)

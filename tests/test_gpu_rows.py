@@ -37,6 +37,10 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
     xd = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(x))
     rd = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(res)) if residual else None
 
+    text = conv.plan(n, n)
+    print(text, flush=True)
+    assert f" rows=512 cols=96 grid=257x{cout // 96} else mfma tiling=19 " in text
+
     def run(m):
         y = s3dx.DeviceArray((n, cout), np.uint16)
         conv.run(xd, n, s3dx.DeviceArray.from_host(m), n, y, s3dx.BF16, rd)
@@ -54,7 +58,7 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
         g, v = (W.bf16_bits_to_f32(t).reshape(t.shape) for t in (got, want))
         rel = float(np.linalg.norm(g - v) / np.linalg.norm(v))
         print(f"{cin}->{cout} {name}: rel-L2 against split-K {rel:.2e}", flush=True)
-        assert 0.0 < rel < 2.0 ** -11  # (0: the kernel did not run)
+        assert 0.0 < rel < 2.0 ** -11
         ref = O.conv(a, m[rows], n, W.round_bf16(w), 1, cout, b)
         ref = O.silu(ref) if silu else ref
         check_rel(g[rows], ref + (res[rows >> 3] if residual else 0.0), 1e-2, "oracle")
@@ -72,7 +76,8 @@ def test_source_rows_above_2_24(s3dx, O, W, monkeypatch):
     one, none = s3dx.DeviceArray.from_host(np.ones(cin, np.float32)), s3dx.DeviceArray.from_host(np.zeros(cin, np.float32))
     conv = s3dx.SparseConv(cin, cout, 27, s3dx.BF16).set_weights(w, s3dx.WEIGHT_MESH, b).set_input_affine_silu(one, none)
     xd, kd, y = s3dx.DeviceArray.from_host(x), s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray((n, cout), np.uint16)
-    print("rows above 2^24", flush=True)
+    print(f"rows above 2^24: {conv.plan(n_in, n)}", flush=True)
+    assert " rows=512 " in conv.plan(n_in, n)
     conv.run(xd, n_in, kd, n, y, s3dx.BF16)
     rows = np.sort(rng.choice(n, 500, replace=False))
     a = W.round_bf16(O.silu(W.bf16_bits_to_f32(x[far:]).reshape(-1, cin)))
