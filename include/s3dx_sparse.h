@@ -383,7 +383,7 @@ S3DX_API s3dx_status s3dx_kmap_subm3_planned(const int32_t *coords, int64_t n, i
  * they run as three BF16 terms where that is faster, deterministic and with no
  * larger error against float64, but rounded differently (within 2e-6); with a
  * plan built for a BF16 layer they ignore it.
- * Launches that do not use the halo kernel ignore the plan. */
+ * Launches that do not read the plan ignore it: they are s3dx_conv_run's. */
 S3DX_API s3dx_status s3dx_conv_run_planned(const s3dx_conv *conv, const s3dx_gather_plan *plan, const void *x,
                                            int64_t n_in, const int32_t *kmap, int64_t n_out, const void *residual,
                                            void *y, int32_t y_dtype, s3dx_stream stream, char *error,

@@ -945,7 +945,7 @@ Route route_of(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const Sourc
     if (r.widen) r.p = plan_launch(conv, count * 4, n_out, aligned16);
     if (xvec) {
         r.fold = fold_blocks_of(conv, r.p, src, n_in, n_out, residual, y_dtype);
-        r.rows = !r.fold && !gplan && rows_of(conv, r.p, src, n_out, y_dtype);
+        r.rows = !r.fold && rows_of(conv, r.p, src, n_out, y_dtype);
         if (r.fold || r.rows) return r;
     }
     if (gplan) {
@@ -956,7 +956,7 @@ Route route_of(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const Sourc
     }
     if (!r.planned) {
         r.whole = r.p;
-        r.own = !gplan && f3_own_plan(conv, r.p, src, n_out);
+        r.own = f3_own_plan(conv, r.p, src, n_out);
     }
     return r;
 }

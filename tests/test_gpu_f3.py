@@ -221,3 +221,18 @@ def test_folded_fp32_maps_and_infinities(s3dx, W, monkeypatch):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and np.isnan(want).any()
     first = _run(s3dx, conv, x, kmap, cout)
     assert rel_l2(first, _ref(h, np.where(kmap >= 0, kmap >> 3, -1), w, b, mesh=True)) < 2e-6
+
+
+def test_a_bf16_layers_plan_changes_nothing(s3dx, W):
+    # A layer with transforms makes records of its own; with a plan that it cannot
+    # read (one made for a BF16 layer) it still does.
+    conv, kmap, x, h, w, b = _mesh(s3dx, W, 2003, 96, 96, False)
+    n = x.shape[0]
+    kd, xd = s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray.from_host(x)
+    other = s3dx.SparseConv(128, 128, 27, s3dx.BF16)
+    gp = other.gather_plan(n, kd, n)
+    assert conv.plan(n, n, gp) == conv.plan(n, n) and conv.plan(n, n).endswith(" plan=own")
+    ys = [s3dx.DeviceArray((n, 96), np.float32) for _ in range(2)]
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32, plan=gp)
+    assert np.array_equal(ys[0].download(), ys[1].download())

@@ -83,3 +83,21 @@ def test_source_rows_above_2_24(s3dx, O, W, monkeypatch):
     a = W.round_bf16(O.silu(W.bf16_bits_to_f32(x[far:]).reshape(-1, cin)))
     ref = O.conv(a, kmap[rows] - far, 40960, W.round_bf16(w), 1, cout, b)
     check_rel(W.bf16_bits_to_f32(y.download()[rows]).reshape(-1, cout), ref, 1e-2, "oracle")
+
+
+def test_a_plan_changes_nothing(s3dx, W):
+    # 512-row tiles read no gather plan: a run that is given one is the same run.
+    parents = W.shells_union(0)[:16421]
+    p, cin = parents.shape[0], 96
+    n = 8 * p
+    _, kd = s3dx.subdivide2(s3dx.DeviceArray.from_host(parents), p, True)
+    x = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(W.normal_f32(140, 1, (n, cin))))
+    one, none = s3dx.DeviceArray.from_host(np.ones(cin, np.float32)), s3dx.DeviceArray.from_host(np.zeros(cin, np.float32))
+    conv = (s3dx.SparseConv(cin, cin, 27, s3dx.BF16).set_weights(W.conv_weight(140, 2, cin, cin, layout="mesh"), s3dx.WEIGHT_MESH, None)
+            .set_input_affine_silu(one, none))
+    gp = conv.gather_plan(n, kd, n)
+    assert conv.plan(n, n, gp) == conv.plan(n, n) and " rows=512 " in conv.plan(n, n)
+    ys = [s3dx.DeviceArray((n, cin), np.uint16) for _ in range(2)]
+    conv.run(x, n, kd, n, ys[0], s3dx.BF16)
+    conv.run(x, n, kd, n, ys[1], s3dx.BF16, plan=gp)
+    assert np.array_equal(ys[0].download(), ys[1].download())
