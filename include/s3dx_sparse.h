@@ -343,9 +343,10 @@ S3DX_API s3dx_status s3dx_conv_run(const s3dx_conv *conv, const void *x, int64_t
  * in use.  create enqueues the build on `stream` and picks the records' tile
  * height from `conv`: 128 output rows when its halo kernel's 128-row tiles
  * fill the GPU's compute units in one pass (runs then use an 8-wave kernel
- * on those tiles; 18 KiB of device memory per 128 rows), or when it is an
- * FP32 layer that runs as three BF16 terms, else 64 rows (7 KiB per 64
- * rows); free releases it. */
+ * on those tiles; 18 KiB of device memory per 128 rows), else 64 rows (7 KiB
+ * per 64 rows).  An FP32 layer that can run as three BF16 terms adds records of
+ * 128 rows for that to the 64-row ones (without room for them, or above 14.9M
+ * rows, FP32 layers run as without a plan).  free releases it. */
 typedef struct s3dx_gather_plan s3dx_gather_plan;
 S3DX_API s3dx_status s3dx_gather_plan_create(const s3dx_conv *conv, int64_t n_in, const int32_t *kmap,
                                              int64_t n_out, s3dx_stream stream, s3dx_gather_plan **out,
@@ -379,7 +380,7 @@ S3DX_API s3dx_status s3dx_kmap_subm3_planned(const int32_t *coords, int64_t n, i
  * of (tile, 64-channel chunk) units one per CU, and a tile split between
  * runs adds its pieces in a fixed order, so results are deterministic but
  * rounded differently from the unplanned run (within BF16 rounding), and
- * except for FP32 layers: with a 128-row plan last built for an FP32 layer
+ * except for FP32 layers: with a plan created and last built for an FP32 layer
  * they run as three BF16 terms where that is faster, deterministic and with no
  * larger error against float64, but rounded differently (within 2e-6); with a
  * plan built for a BF16 layer they ignore it.

@@ -337,12 +337,18 @@ struct s3dx_conv {
 struct s3dx_gather_plan {
     void *d = nullptr;
     int rows = 64;         // tile height of the records (64 or 128)
-    bool f32 = false;      // built for an FP32 layer: such layers then run as three BF16 terms
-    int64_t capacity = 0;  // output rows the allocation covers
+    // 128-row records beside 64-row ones, where an FP32 layer that can run as
+    // three BF16 terms created the plan: BF16 layers over it read the others.
+    void *d3 = nullptr;
+    bool f32 = false;      // last built for an FP32 layer: the 128-row records are the map's
+    int64_t capacity = 0;  // output rows the allocations cover
     int64_t n_out = 0, n_src = 0;
     int32_t shift = 0;
+    // What an FP32 layer reads as three BF16 terms, or nullptr.
+    void *f3_records() const { return !f32 ? nullptr : d3 ? d3 : rows == 128 ? d : nullptr; }
     ~s3dx_gather_plan() {
         if (d) (void)hipFree(d);
+        if (d3) (void)hipFree(d3);
     }
 };
 
@@ -781,28 +787,32 @@ int f3_blocks(const s3dx_conv *conv, int64_t n_out) {
     return best;
 }
 
+// The launch of an FP32 layer as three BF16 terms over 128-row records of its map,
+// where that pays.
+bool apply_f3(LaunchPlan &p, const s3dx_conv *conv, int64_t n_out) {
+    if (!p.mfma || !p.tl || p.xf || !f3_shape(conv) || (!conv->w3 && conv->weights_set) || std::getenv("S3DX_CONV_TILING"))
+        return false;
+    const int cg = f3_blocks(conv, n_out);
+    if (!cg) return false;
+    for (const Tiling &t : kTilings)
+        if (t.id == 25) p.tl = &t;
+    p.f3 = p.nb = cg;
+    p.kc = 32;
+    p.fn = pick_f3(cg);
+    p.threads = kHalo8Threads;
+    p.stream_k = p.sk_splitk = false;
+    p.fused_ln = conv->ln && cg * 32 == conv->cout;
+    p.grid = dim3(static_cast<unsigned>((n_out + 127) / 128), static_cast<unsigned>(conv->cout_pad / 32 / cg));
+    return true;
+}
+
 // A planned launch: the halo kernel of the plan's tile height in place of
 // the unplanned halo kernel (64-row records: tiling 21 only; 128-row records:
-// tilings 20 and 21, on the 8-wave kernel, in stream-K runs where those pay).
-// Other launches are unchanged.
+// tilings 20 and 21, on the 8-wave kernel, in stream-K runs where those pay), or
+// an FP32 layer as three BF16 terms.  Other launches are unchanged.
 void apply_gather_plan(LaunchPlan &p, const s3dx_conv *conv, const s3dx_gather_plan *g, int64_t n_out, bool bf16_rows) {
     const int cin = conv->cin;
-    if (!bf16_rows && p.mfma && p.tl && !p.xf && g->f32 && g->rows == 128 && f3_shape(conv) &&
-        (conv->w3 || !conv->weights_set) && !std::getenv("S3DX_CONV_TILING")) {
-        const int cg = f3_blocks(conv, n_out);
-        if (cg) {
-            for (const Tiling &t : kTilings)
-                if (t.id == 25) p.tl = &t;
-            p.f3 = p.nb = cg;
-            p.kc = 32;
-            p.fn = pick_f3(cg);
-            p.threads = kHalo8Threads;
-            p.stream_k = p.sk_splitk = false;
-            p.fused_ln = conv->ln && cg * 32 == conv->cout;
-            p.grid = dim3(static_cast<unsigned>((n_out + 127) / 128), static_cast<unsigned>(conv->cout_pad / 32 / cg));
-            return;
-        }
-    }
+    if (!bf16_rows && g->f3_records() && apply_f3(p, conv, n_out)) return;
     if (bf16_rows || !p.mfma || !p.tl || (p.tl->id != 20 && p.tl->id != 21)) return;
     if (g->rows == 64 && p.tl->id == 21) {
         p.fn = pick_halo_bf16_planned(64, p.nb);
@@ -830,11 +840,15 @@ bool f3_own_plan(const s3dx_conv *conv, LaunchPlan &p, const Source &src, int64_
     if (!src.pre || conv->dtype != S3DX_F32 || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
         (n_out + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31) || n_out < 8192)
         return false;
-    s3dx_gather_plan g;
-    g.rows = 128;
-    g.f32 = true;
-    apply_gather_plan(p, conv, &g, n_out, false);
-    return p.f3 != 0;
+    return apply_f3(p, conv, n_out);
+}
+
+// Whether a gather plan for `conv` also holds 128-row records for the three-term
+// kernel (below 2 GiB, as its offsets into them).
+bool gather_plan_f3(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
+    if ((n_out + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31)) return false;
+    LaunchPlan p = plan_launch(conv, x_bytes, n_out, true);
+    return apply_f3(p, conv, n_out);
 }
 
 // Tile height of the gather plan for `conv`: 128-row records when the
@@ -846,7 +860,6 @@ int gather_plan_rows(const s3dx_conv *conv, int64_t x_bytes, int64_t n_out) {
         if (r == 64 || r == 128) return r;
     }
     const LaunchPlan p = plan_launch(conv, x_bytes, n_out, true);
-    if (f3_shape(conv) && p.mfma && p.tl && !p.xf && !std::getenv("S3DX_CONV_TILING") && f3_blocks(conv, n_out)) return 128;
     if (!p.mfma || !p.tl || (p.tl->id != 20 && p.tl->id != 21) || p.nb != 4 || p.half_chunk) return 64;
     const int64_t tiles = (n_out + 127) / 128 * static_cast<int64_t>(p.grid.y);
     return tiles <= device_cus() || stream_k_runs(conv->cin, n_out, p.grid.y) ? 128 : 64;
@@ -1374,7 +1387,7 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
                           conv->cout / 96);
         std::snprintf(plan, plan_capacity, "%s%s%s%s%s%s", bf16_rows ? (r.widen ? "in=bf16 pre=widen " : "in=bf16 ") : "",
                       src.pre ? (src.children ? "pre=children " : "pre=rows ") : "", src.shift ? "parent-rows " : "",
-                      most, text, r.planned ? (gplan->rows == 128 ? " plan=128" : " plan=64") : r.own ? " plan=own" : "");
+                      most, text, r.planned ? (gplan->rows == 128 || p.f3 ? " plan=128" : " plan=64") : r.own ? " plan=own" : "");
     }
 }
 
@@ -1507,7 +1520,7 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             a.x_bytes = count * 4;
         }
         if (plan.split) a.w = conv->w_split;
-        if (route.planned) a.plan = gplan->d;
+        if (route.planned) a.plan = plan.f3 ? gplan->f3_records() : gplan->d;
         if (plan.f3) a.w3 = conv->w3;
         if (fold) {
             launch_fold_plan(kmap, n_in, fold_records, fold_state, !bf, s);
@@ -1607,6 +1620,20 @@ S3DX_API s3dx_status s3dx_conv_run(const s3dx_conv *conv, const void *x, int64_t
 
 namespace {
 
+// The rest of a build once d's records are enqueued: the FP32 layers' records, and
+// what the plan is of.
+void gather_plan_built(s3dx_gather_plan *p, const s3dx_conv *conv, const int32_t *kmap, int64_t n_out, int64_t n_src,
+                       int32_t shift, s3dx_stream stream) {
+    p->f32 = conv->dtype == S3DX_F32;
+    if (p->f32 && p->d3) {
+        launch_gather_plan_build(128, kmap, n_out, n_src, shift, p->d3, as_stream(stream));
+        launch_check("gather_plan_build");
+    }
+    p->n_out = n_out;
+    p->n_src = n_src;
+    p->shift = shift;
+}
+
 // Checks the arguments and enqueues the build of `p` (allocated for at least
 // n_out rows) over `kmap`.
 void gather_plan_build(s3dx_gather_plan *p, const s3dx_conv *conv, int64_t n_in, const int32_t *kmap,
@@ -1617,10 +1644,7 @@ void gather_plan_build(s3dx_gather_plan *p, const s3dx_conv *conv, int64_t n_in,
     require(n_out * kMaxKvol * 4 < (int64_t(1) << 31), "kernel maps of 2 GiB or more have no gather plan");
     launch_gather_plan_build(p->rows, kmap, n_out, src.n_src, src.shift, p->d, as_stream(stream));
     launch_check("gather_plan_build");
-    p->n_out = n_out;
-    p->n_src = src.n_src;
-    p->shift = src.shift;
-    p->f32 = conv->dtype == S3DX_F32;
+    gather_plan_built(p, conv, kmap, n_out, src.n_src, src.shift, stream);
 }
 
 void gather_plan_check(const s3dx_conv *conv, int64_t n_in, const int32_t *kmap, int64_t n_out) {
@@ -1643,12 +1667,17 @@ S3DX_API s3dx_status s3dx_gather_plan_create(const s3dx_conv *conv, int64_t n_in
         gather_plan_check(conv, n_in, kmap, n_out);
         const Source src = source_of(conv, n_in);
         auto p = std::make_unique<s3dx_gather_plan>();
-        p->rows = gather_plan_rows(conv, src.rows * conv->cin * static_cast<int64_t>(dtype_size(conv->in_dtype)),
-                                   n_out);
+        const int64_t x_bytes = src.rows * conv->cin * static_cast<int64_t>(dtype_size(conv->in_dtype));
+        p->rows = gather_plan_rows(conv, x_bytes, n_out);
         const int64_t bytes =
             (n_out + p->rows - 1) / p->rows * (p->rows == 128 ? kGatherPlanRecord128 : kGatherPlanRecord);
         require(bytes < (int64_t(1) << 31), "map too large for a gather plan");
         hip_check(hipMalloc(&p->d, static_cast<size_t>(bytes)), "hipMalloc gather plan");
+        if (p->rows == 64 && gather_plan_f3(conv, x_bytes, n_out) &&
+            hipMalloc(&p->d3, static_cast<size_t>((n_out + 127) / 128 * kGatherPlanRecord128)) != hipSuccess) {
+            (void)hipGetLastError();  // no room: FP32 layers run on FP32 matrix instructions
+            p->d3 = nullptr;
+        }
         p->capacity = n_out;
         gather_plan_build(p.get(), conv, n_in, kmap, n_out, stream);
         *out = p.release();
@@ -1682,10 +1711,7 @@ S3DX_API s3dx_status s3dx_kmap_subm3_planned(const int32_t *coords, int64_t n, i
         launch_kmap_plan(plan->rows, coords, n, missing_value, kmap, workspace, workspace_bytes, plan->d,
                          as_stream(stream));
         launch_check("kmap_plan");
-        plan->n_out = n;
-        plan->n_src = n;
-        plan->shift = 0;
-        plan->f32 = conv->dtype == S3DX_F32;
+        gather_plan_built(plan, conv, kmap, n, n, 0, stream);
     });
 }
 

@@ -236,3 +236,32 @@ def test_a_bf16_layers_plan_changes_nothing(s3dx, W):
     conv.run(xd, n, kd, n, ys[0], s3dx.F32)
     conv.run(xd, n, kd, n, ys[1], s3dx.F32, plan=gp)
     assert np.array_equal(ys[0].download(), ys[1].download())
+
+
+@pytest.mark.parametrize("n,cin,cout", [(12801, 128, 128), (12801, 128, 96), (28265, 256, 512), (10366, 128, 128)])
+def test_bf16_layers_over_an_fp32_layers_plan(s3dx, O, W, n, cin, cout):
+    # A plan that an FP32 layer made serves BF16 layers as a 64-row plan does.
+    coords = W.shells_union(0)[:n]
+    kd = s3dx.kmap_subm3(s3dx.DeviceArray.from_host(coords), n, n)
+    gp = s3dx.SparseConv(128, 128, 27, s3dx.F32).gather_plan(n, kd, n)
+    conv = s3dx.SparseConv(cin, cout, 27, s3dx.BF16).set_weights(W.conv_weight(150, 1, cin, cout), s3dx.WEIGHT_SLAT, None)
+    cols = 128 if cout % 128 == 0 else 96
+    text = conv.plan(n, n, gp)
+    assert text.startswith(f"mfma tiling=21 split-k halo rows=64 cols={cols} ") and text.endswith(" plan=64"), text
+    x = s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(W.normal_f32(150, 2, (n, cin))))
+    ys = [s3dx.DeviceArray((n, cout), np.uint16) for _ in range(2)]
+    conv.run(x, n, kd, n, ys[0], s3dx.BF16)
+    conv.run(x, n, kd, n, ys[1], s3dx.BF16, plan=gp)
+    assert np.array_equal(ys[0].download(), ys[1].download())
+
+
+def test_plan_of_a_map_too_long_for_128_row_records(s3dx, W):
+    # 15.5M rows: 2.2 GB of 128-row records, whose offsets have 31 bits; the plan is
+    # made with the 64-row ones alone, and the FP32 layer ignores it.
+    n = 15_500_000
+    kd = s3dx.DeviceArray.from_host(np.zeros((n, 27), np.int32))
+    conv = s3dx.SparseConv(32, 32, 27, s3dx.F32)
+    print("plan of 15.5M rows", flush=True)
+    gp = conv.gather_plan(n, kd, n)
+    assert "terms=3" not in conv.plan(n, n, gp)
+    s3dx.synchronize()
