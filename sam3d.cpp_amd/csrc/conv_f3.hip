@@ -26,8 +26,10 @@
 // holds a partial sum of another's outputs (with KS 1).
 //
 // Tiles that name more rows than the planes hold (719; a union of sphere
-// shells names about 470 in 128 rows, 534 at most) gather them from memory and
-// split them in registers.  Tiles whose rows hold a value with no finite first
+// shells names about 470 in 128 rows, 534 at most, a solid bar of 24 x 24 x 60 up
+// to 768) are multiplied in two parts.  Tiles without slots (rows in no order) stage
+// five offsets' rows at a time, or, with fewer than 128 columns a workgroup, gather
+// rows from memory and split them in registers.  Tiles whose rows hold a value with no finite first
 // term (infinities, NaN) are done again with FP32 matrix instructions, so that
 // such values spread as in any FP32 sum.
 #include "halo_tile.hpp"
@@ -36,7 +38,12 @@ namespace s3dx {
 namespace {
 
 constexpr int kF3Chunk = 32;                               // channels per chunk
+constexpr int kF3MostRows = 719;                           // distinct rows that it stages at once
+constexpr int kF3Part = 712;                               // of more, the first (whole swizzle periods, one row fewer)
 constexpr int kF3Rows = kF3MostRows + 1;                   // rows a plane holds (the last is the zero row)
+constexpr int kF3Offsets = 5;                              // offsets of 128 rows that it stages at once
+static_assert(kF3Part % 8 == 0 && kF3Part < kF3MostRows && kH8Single - kF3Part < kF3Part, "two parts");
+static_assert(kF3Offsets * 128 <= kF3MostRows, "five offsets' rows");
 constexpr int kF3Plane = kF3Rows * kF3Chunk * 2;           // bytes of one term's plane
 constexpr int kF3Rec = 3 * kF3Plane;                       // the plan record, behind the planes
 constexpr int kF3Flag = kF3Rec + kGatherPlanRecord128;     // a row held a value without terms
@@ -131,8 +138,13 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
     const uint32_t mode = __builtin_amdgcn_readfirstlane(hdr[0]);
     const int distinct = static_cast<int>(__builtin_amdgcn_readfirstlane(hdr[1]));
     const uint32_t mask = __builtin_amdgcn_readfirstlane(hdr[2]);
-    const bool staged = mode == 0u && distinct < kF3Rows;
-    if (FOLD && !staged) return;  // a listed tile
+    if (FOLD && mode != 0u) return;  // a listed tile
+    // What the planes hold at a time (a pass over a chunk): the tile's distinct
+    // rows; of more than they have room for, the first kF3Part, then the rest; in a
+    // tile without slots (mode 1) the 128 rows that each of five offsets names.
+    const bool slots = FOLD || mode == 0u;
+    const int passes = slots ? (distinct > kF3MostRows ? 2 : 1) : (__popc(mask) + kF3Offsets - 1) / kF3Offsets;
+    const int width = passes > 1 ? kF3Part : kF3MostRows;  // distinct rows a pass
 
     const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.x), static_cast<short>(0),
                                                           static_cast<int32_t>(a.x_bytes), 0x00020000);
@@ -161,27 +173,74 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
             for (uint32_t r = mask; r != 0u; r &= r - 1u, ++k)
                 if ((k & 1) == (kp >> 1)) mine |= r & (0u - r);
         }
-        const int n = __popc(mine);
-        const int olast = n > 0 ? 31 - __builtin_clz(mine) : 0;
+        // The table entry of row block mb of this wave's rows at offset o.
+        auto entry = [&](int o, int mb) __attribute__((always_inline)) {
+            return table[o * ROWS + rg * 64 + mb * 32 + (lane & 31)];
+        };
+        // Mode 1: the offsets of pass q.
+        auto group = [&](int q) __attribute__((always_inline)) {
+            uint32_t rest = mask;
+            for (int k = 0; k < q * kF3Offsets; ++k) rest &= rest - 1u;
+            uint32_t after = rest;
+            for (int k = 0; k < kF3Offsets; ++k) after &= after - 1u;
+            return rest & ~after;
+        };
+        // The wave's offsets in the two passes over slots: those that name one of
+        // the pass's rows (of the next plane of the set few offsets do, so that the
+        // second pass is a short one).
+        uint32_t part[2] = {mine, mine};
+        if (slots && passes > 1) {
+            part[0] = part[1] = 0u;
+            for (uint32_t r = mine; r != 0u; r &= r - 1u) {
+                const int o = __builtin_ctz(r);
+                bool first = false, second = false;
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) {
+                    const int sl = static_cast<int>(entry(o, mb) >> 7);
+                    first = first || sl < kF3Part;
+                    second = second || (sl >= kF3Part && sl < distinct);
+                }
+                if (__builtin_amdgcn_ballot_w64(first)) part[0] |= r & (0u - r);
+                if (__builtin_amdgcn_ballot_w64(second)) part[1] |= r & (0u - r);
+            }
+        }
+        uint32_t cur = mine;  // the wave's offsets in this pass, and the last of them
+        int olast = 0;
         auto advance = [&](uint32_t &rest) __attribute__((always_inline)) {
             const int o = __builtin_ctz(rest | 0x80000000u);
             rest &= rest - 1u;
             return o == 31 ? olast : o;
         };
-        // A chunk's rows: piece i of a thread is channels 4j .. 4j + 3 of slot
+        // A pass's rows: piece i of a thread is channels 4j .. 4j + 3 of place
         // 64 i + tid / 8, j = tid % 8 (eight lanes read a row's 128 bytes).
         constexpr int XP = (kF3Rows + 63) / 64;  // 12
         u32x4 xq[XP];
-        auto load_x = [&](int c) __attribute__((always_inline)) {
+        auto load_x = [&](auto by_slot, int c, int q) __attribute__((always_inline)) {
+            // (24-bit products: rows of at least 128 bytes, x below 2 GiB; the top
+            // bit, set last: past the rows, zeros)
+            const uint32_t p16 = (tid & 7) * 16u;
+            uint32_t off[XP];
+            if constexpr (by_slot.value) {
 #pragma unroll
-            for (int i = 0; i < XP; ++i) {
-                const int sl = 64 * i + (tid >> 3);
-                // (24 bits: rows of at least 128 bytes, x below 2 GiB)
-                const uint32_t off = (__umul24(slot_row[min(sl, kF3Rows - 1)], 4u * static_cast<uint32_t>(a.cin)) +
-                                      (tid & 7) * 16u) |
-                                     (sl < distinct ? 0u : 0x80000000u);  // past the rows: zeros
-                xq[i] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, static_cast<int32_t>(off), c * (kF3Chunk * 4), 0);
+                for (int i = 0; i < XP; ++i) {
+                    const int at = 64 * i + (tid >> 3), sl = at + q * kF3Part;
+                    off[i] = (__umul24(slot_row[min(sl, kH8Single - 1)], 4u * static_cast<uint32_t>(a.cin)) + p16) |
+                             (at < width && sl < distinct ? 0u : 0x80000000u);
+                }
+            } else {
+                uint32_t rest = group(q);
+#pragma unroll
+                for (int i = 0; i < XP; ++i) {
+                    const int o = __builtin_ctz(rest | 0x80000000u);
+                    const uint32_t row = table[min(o, kMaxKvol - 1) * ROWS + 64 * (i & 1) + (tid >> 3)];
+                    off[i] = (__umul24(row, 4u * static_cast<uint32_t>(a.cin)) + p16) |
+                             (o < kMaxKvol && static_cast<int32_t>(row) >= 0 ? 0u : 0x80000000u);
+                    if (i & 1) rest &= rest - 1u;
+                }
             }
+#pragma unroll
+            for (int i = 0; i < XP; ++i)
+                xq[i] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, static_cast<int32_t>(off[i]), c * (kF3Chunk * 4), 0);
         };
         auto store_x = [&](char *p) __attribute__((always_inline)) {
 #pragma unroll
@@ -216,15 +275,28 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
                 b[t] = make_uint4(v.x, v.y, v.z, v.w);
             }
         };
-        // the record's offsets are 128-byte ones (slot * 128 | swizzle): the
-        // slot's 64 bytes and this kernel's swizzle from the same bits.  A
-        // missing neighbour is the record's zero slot, 559 (past the rows of
-        // the tiles that use it: zeros) or 1088, this kernel's last.
-        auto load_ix = [&](int o) __attribute__((always_inline)) {
+        // The record's offsets are 128-byte ones (slot * 128 | swizzle): the
+        // slot's 64 bytes and this kernel's swizzle from the same bits (kF3Part
+        // slots keep the swizzle).  A missing neighbour is the record's zero slot,
+        // 559 or 1088, past the rows of every tile that uses it: zeros; a slot of the
+        // other pass is the place after this pass's, zeros too, as is the last row.
+        uint32_t base = 0;   // bytes of the slots before this pass's
+        uint32_t grp = 0;    // mode 1: the pass's offsets
+        const uint32_t limit = static_cast<uint32_t>(passes > 1 ? kF3Part : kF3Rows - 1) * 64u;
+        auto load_ix = [&](auto by_slot, int o) __attribute__((always_inline)) {
+            if constexpr (by_slot.value) {
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-                const uint32_t v = table[o * ROWS + rg * 64 + mb * 32 + (lane & 31)];
-                ix[mb] = min((v >> 1) & ~63u, (kF3Rows - 1) * 64u) | (((v >> 4) & 0x30u) ^ (half << 4));
+                for (int mb = 0; mb < 2; ++mb) {
+                    const uint32_t v = entry(o, mb);
+                    ix[mb] = min(((v >> 1) & ~63u) - base, limit) | (((v >> 4) & 0x30u) ^ (half << 4));
+                }
+            } else {
+                const int j = __popc(grp & ((1u << o) - 1u));
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) {
+                    const int at = min(j, kF3Offsets - 1) * ROWS + rg * 64 + mb * 32 + (lane & 31);
+                    ix[mb] = static_cast<uint32_t>(at * 64 + ((((at >> 1) & 3) ^ half) << 4));
+                }
             }
         };
         auto load_a = [&](const char *p, int k, uint4 (&af)[2][3]) __attribute__((always_inline)) {
@@ -248,14 +320,76 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb) hi[mb] = mfma_step<uint16_t>(af[mb][0], b[0], hi[mb]);
         };
-        // The source row of this lane's row of block mb at offset o, or -1.
-        auto row_of = [&](int o, int mb) __attribute__((always_inline)) {
-            const uint32_t v = table[o * ROWS + rg * 64 + mb * 32 + (lane & 31)];
-            const int sl = static_cast<int>(v >> 7);
-            return mode != 0u ? static_cast<int32_t>(v)
-                              : sl < distinct ? static_cast<int32_t>(slot_row[min(sl, kH8Single - 1)]) : -1;
+        auto multiply = [&](auto by_slot) __attribute__((always_inline)) {
+            load_x(by_slot, 0, 0);
+            for (int c = 0, q = 0; c < chunks;) {
+                if constexpr (!by_slot.value) grp = group(q);
+                cur = by_slot.value ? part[q] : mine & grp;
+                olast = cur != 0u ? 31 - __builtin_clz(cur) : 0;
+                base = static_cast<uint32_t>(q) * (kF3Part * 64u);
+                const int n = __popc(cur);
+                const int qn = q + 1 < passes ? q + 1 : 0, cn = qn ? c : c + 1;
+                // the pass's first weights, in flight while its rows are split
+                uint32_t rest_b = cur, rest_i = cur;
+                if constexpr (KS == 1) {
+                    const int o = advance(rest_b);
+                    load_b(c, o, 0, bq[0]);
+                    load_b(c, o, 1, bq[1]);
+                } else {
+                    load_b(c, advance(rest_b), kp & 1, bq[0]);
+                    load_b(c, advance(rest_b), kp & 1, bq[1]);
+                }
+                if (c + q > 0) __syncthreads();  // every wave is done with the planes
+                store_x(planes);
+                __syncthreads();
+                if (cn < chunks) load_x(by_slot, cn, qn);
+                sched_fence();
+                load_ix(by_slot, advance(rest_i));
+                if constexpr (KS == 1) {
+                    load_a(planes, 0, aq[0]);
+                    for (int i = 0; i < n; ++i) {
+                        const int o = advance(rest_b);
+                        load_a(planes, 1, aq[1]);
+                        load_ix(by_slot, advance(rest_i));
+                        products(aq[0], bq[0]);
+                        sched_fence();
+                        load_b(c, o, 0, bq[0]);
+                        load_a(planes, 0, aq[0]);
+                        products(aq[1], bq[1]);
+                        sched_fence();
+                        load_b(c, o, 1, bq[1]);
+                    }
+                } else {
+                    const int k = kp & 1;
+                    load_a(planes, k, aq[0]);
+                    load_ix(by_slot, advance(rest_i));
+                    int i = 0;
+                    for (; i + 2 <= n; i += 2) {
+                        load_a(planes, k, aq[1]);
+                        load_ix(by_slot, advance(rest_i));
+                        products(aq[0], bq[0]);
+                        sched_fence();
+                        load_b(c, advance(rest_b), k, bq[0]);
+                        load_a(planes, k, aq[0]);
+                        load_ix(by_slot, advance(rest_i));
+                        products(aq[1], bq[1]);
+                        sched_fence();
+                        load_b(c, advance(rest_b), k, bq[1]);
+                    }
+                    if (i < n) products(aq[0], bq[0]);
+                }
+                c = cn;
+                q = qn;
+            }
         };
-        if (!FOLD && !staged) {
+        if (slots) {
+            multiply(std::true_type{});
+        } else if constexpr (KS == 1 && !FOLD) {
+            multiply(std::false_type{});
+        } else if constexpr (KS > 1) {
+            // (with fewer columns a workgroup, staging five offsets' rows takes longer
+            // than their products: 192 -> 192 on 65,536 shuffled rows 1,181 us against
+            // 943, 64 -> 64 on 28,265 80 against 66)
             // Rows from memory, split in registers: channels 16 k + 8 half .. + 7
             // of the lane's row for every (offset, k-step) of this wave.
             uint4 raw[2][2][2];  // [set][row block][16-byte half]
@@ -285,7 +419,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
             // k-steps kp, kp + KS, ... of the layer's
             for (uint32_t rest = mask; rest != 0u; rest &= rest - 1u) {
                 const int o = __builtin_ctz(rest);
-                const int32_t row[2] = {row_of(o, 0), row_of(o, 1)};
+                const int32_t row[2] = {static_cast<int32_t>(entry(o, 0)), static_cast<int32_t>(entry(o, 1))};
                 if (kp < ksteps) {
                     load_raw(row, kp, raw[0]);
                     load_b(0, o, kp, bq[0]);
@@ -307,58 +441,6 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
                     split_raw(raw[0], aq[0]);
                     products(aq[0], bq[0]);
                 }
-            }
-        }
-        if (staged) load_x(0);
-        for (int c = 0; staged && c < chunks; ++c) {
-            // the chunk's first weights, in flight while its rows are split
-            uint32_t rest_b = mine, rest_i = mine;
-            if constexpr (KS == 1) {
-                const int o = advance(rest_b);
-                load_b(c, o, 0, bq[0]);
-                load_b(c, o, 1, bq[1]);
-            } else {
-                load_b(c, advance(rest_b), kp & 1, bq[0]);
-                load_b(c, advance(rest_b), kp & 1, bq[1]);
-            }
-            if (c > 0) __syncthreads();  // every wave is done with the planes
-            store_x(planes);
-            __syncthreads();
-            if (c + 1 < chunks) load_x(c + 1);
-            sched_fence();
-            load_ix(advance(rest_i));
-            if constexpr (KS == 1) {
-                load_a(planes, 0, aq[0]);
-                for (int i = 0; i < n; ++i) {
-                    const int o = advance(rest_b);
-                    load_a(planes, 1, aq[1]);
-                    load_ix(advance(rest_i));
-                    products(aq[0], bq[0]);
-                    sched_fence();
-                    load_b(c, o, 0, bq[0]);
-                    load_a(planes, 0, aq[0]);
-                    products(aq[1], bq[1]);
-                    sched_fence();
-                    load_b(c, o, 1, bq[1]);
-                }
-            } else {
-                const int k = kp & 1;
-                load_a(planes, k, aq[0]);
-                load_ix(advance(rest_i));
-                int i = 0;
-                for (; i + 2 <= n; i += 2) {
-                    load_a(planes, k, aq[1]);
-                    load_ix(advance(rest_i));
-                    products(aq[0], bq[0]);
-                    sched_fence();
-                    load_b(c, advance(rest_b), k, bq[0]);
-                    load_a(planes, k, aq[0]);
-                    load_ix(advance(rest_i));
-                    products(aq[1], bq[1]);
-                    sched_fence();
-                    load_b(c, advance(rest_b), k, bq[1]);
-                }
-                if (i < n) products(aq[0], bq[0]);
             }
         }
         if (none) *flag = 1u;

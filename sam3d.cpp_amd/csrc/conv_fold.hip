@@ -473,7 +473,7 @@ void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t
 void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, bool f32, hipStream_t stream) {
     hipLaunchKernelGGL(fold_plan_kernel, dim3(static_cast<unsigned>((n_parents + 127) / 128)),
                        dim3(kPlanBuild128Threads), 0, stream, kmap, n_parents, static_cast<char *>(plan), state,
-                       f32 ? kF3MostRows : kH8Double);
+                       f32 ? kH8Single : kH8Double);
 }
 
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream) {

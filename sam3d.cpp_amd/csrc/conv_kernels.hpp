@@ -117,7 +117,6 @@ constexpr int kGatherPlanRecord128 = 18432;  // 128-row tiles
 int64_t f3_weight_bytes(int cin, int cout_pad);
 void launch_f3_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
 KernelFn pick_f3(int cg);
-constexpr int kF3MostRows = 719;  // distinct rows of a tile that it stages
 // The same for folded parent rows: the folded weights' terms, and the folded
 // run with the FP32 pass over the listed tiles behind it.
 int64_t f3_fold_weight_bytes(int cin, int cout_pad);

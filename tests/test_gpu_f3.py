@@ -6,7 +6,10 @@ product are accumulated in FP32.  Their error against float64 must not exceed
 the FP32 matrix instructions' on the same inputs (measured: a quarter to nine
 tenths of it), and the FP32 gate (rel-L2 1e-5) holds far off.  Rows in LDS (up
 to 719 distinct ones in a tile), rows gathered from memory, and infinities or
-NaN, which take FP32 matrix instructions, are all reached.
+NaN, which take FP32 matrix instructions, are all reached.  Tiles of more distinct
+rows than the LDS holds (719) are multiplied in two parts, tiles that the plan
+keeps no slots for by five offsets' rows at a time (128 columns a workgroup) or
+from memory.
 """
 import numpy as np
 import pytest
@@ -43,6 +46,11 @@ def _shuffled(c):
     return np.ascontiguousarray(c[np.random.default_rng(5).permutation(len(c))])
 
 
+def _box(x, y, z):
+    g = np.stack(np.meshgrid(np.arange(x), np.arange(y), np.arange(z), indexing="ij"), -1).reshape(-1, 3) + 2
+    return np.ascontiguousarray(np.concatenate([np.zeros((len(g), 1), np.int64), g], 1).astype(np.int32))
+
+
 CASES = {
     # name: (coords, cin, cout, LayerNorm, columns a workgroup)
     "whole_row_ln": (lambda W: W.shells_union(0)[:12801], 128, 128, True, 128),
@@ -51,7 +59,13 @@ CASES = {
     "wide_separate_ln": (lambda W: W.shells_union(2)[:6001], 96, 256, True, None),
     "two_places": (lambda W: _regions(W.shells_union(0)[:12800], 2), 64, 128, False, None),    # 560 to 719 rows
     "four_places": (lambda W: _regions(W.shells_union(0)[:12800], 4), 64, 128, False, None),   # around 719
-    "eight_places": (lambda W: _regions(W.shells_union(0)[:12800], 8), 96, 64, False, None),   # above: from memory
+    "eight_places": (lambda W: _regions(W.shells_union(0)[:12800], 8), 96, 64, False, None),   # above: two parts
+    "solid_box": (lambda W: _box(22, 22, 22), 64, 128, False, None),                           # about 560 rows
+    "solid_bar": (lambda W: _box(16, 24, 60), 64, 128, False, 128),                            # up to 750: two parts
+    "solid_bar_two_k": (lambda W: _box(12, 15, 60), 64, 192, False, 64),
+    "solid_bar_four_k": (lambda W: _box(12, 24, 60), 64, 96, False, 32),
+    "shuffled_two_k": (lambda W: _shuffled(W.shells_union(0)[:9000]), 64, 192, False, 64),
+    "shuffled_four_k": (lambda W: _shuffled(W.shells_union(0)[:9000]), 64, 96, False, 32),
     "shuffled": (lambda W: _shuffled(W.shells_union(0)[:12000]), 64, 128, False, None),        # the plan's global tiles
     "isolated_points": (lambda W: _points(3), 128, 128, False, None),                          # one offset
 }
@@ -198,6 +212,22 @@ def test_layers_with_transforms(s3dx, W, monkeypatch, p, cin, cout, parent):
     e, f = rel_l2(got, ref), rel_l2(fp32, ref)
     print(f"  rel-L2 {e:.2e}, FP32 {f:.2e}", flush=True)
     assert e <= 1.05 * f and e < 2e-6, (e, f)
+
+
+@pytest.mark.parametrize("shape", [(6, 24, 64), (16, 24, 60)])
+def test_folded_solid_sets(s3dx, O, W, monkeypatch, shape):
+    # Solid sets name more than 719 parents in a tile: two parts.
+    parents = _box(*shape)
+    monkeypatch.setattr(W, "shells_union", lambda seed: parents)
+    p, cin, cout = parents.shape[0], 64, 96
+    km = O.kmap_subm3(parents, p)
+    most = max(len(np.unique(km[i:i + 128][km[i:i + 128] < p])) for i in range(0, p, 128))
+    conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, True)
+    print(f"{shape}: {most} rows in a tile; {conv.plan(p, 8 * p)}", flush=True)
+    assert most > 719 and " fold terms=3 " in conv.plan(p, 8 * p)
+    ref = _ref(h, np.where(kmap >= 0, kmap >> 3, -1), w, b, mesh=True)
+    got = _run(s3dx, conv, x, kmap, cout)
+    assert rel_l2(got, ref) < 2e-6 and np.max(np.abs(got - ref)) < 1e-5 * np.max(np.abs(ref))
 
 
 def test_folded_fp32_maps_and_infinities(s3dx, W, monkeypatch):
