@@ -65,7 +65,7 @@ struct XformArgs {
     int32_t children;  // output row r reads x row r >> 3 and adds slot_offset[r & 7]
     const float *slot_offset;
     const float *scale, *shift;
-    uint32_t *fold_state;  // folded runs: the tile count to clear, the flag for infinities and NaN
+    uint32_t *fold_state;  // folded runs: the flag for infinities and NaN
 };
 
 template <class T>
@@ -84,7 +84,6 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
     constexpr int E = 16 / sizeof(T);
     const uint32_t ppr = static_cast<uint32_t>(a.cin) / E;
     const uint32_t total = static_cast<uint32_t>(a.rows) * ppr;
-    if (a.fold_state && blockIdx.x == 0 && threadIdx.x == 0) a.fold_state[kFoldCount] = 0u;
     for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < total; u += gridDim.x * 256u) {
         const uint32_t r = u / ppr;
         const int32_t c0 = static_cast<int32_t>(u - r * ppr) * E;
@@ -934,7 +933,7 @@ bool xvec_of(const s3dx_conv *conv, const Source &src) {
 // alone; shared by s3dx_conv_run and s3dx_conv_plan.
 struct Route {
     LaunchPlan p;          // the kernel; with fold or rows the one for the tiles they leave over
-    LaunchPlan whole;      // own: the kernel without the records
+    LaunchPlan whole;      // fold, rows, own: the kernel of a run that has no room for records
     int fold = 0;          // folded parent rows: 32-column blocks per workgroup
     bool rows = false;     // 512-row tiles
     bool planned = false;  // the kernel reads the caller's gather plan
@@ -959,7 +958,27 @@ Route route_of(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const Sourc
     if (xvec) {
         r.fold = fold_blocks_of(conv, r.p, src, n_in, n_out, residual, y_dtype);
         r.rows = !r.fold && rows_of(conv, r.p, src, n_out, y_dtype);
-        if (r.fold || r.rows) return r;
+        if (r.fold || r.rows) {
+            // the kernels of the tiles left over (launch_*_left)
+            r.whole = r.p;
+            const int blocks = conv->cout_pad / 32;
+            auto take = [&](int id, int nb, int kc) {
+                for (const Tiling &t : kTilings)
+                    if (t.id == id) r.p.tl = &t;
+                r.p.nb = nb;
+                r.p.kc = kc;
+                r.p.stream_k = r.p.sk_splitk = r.p.fused_ln = false;
+                r.p.grid = dim3(static_cast<unsigned>((n_out + r.p.tl->rows() - 1) / r.p.tl->rows()),
+                                static_cast<unsigned>(blocks / nb));
+            };
+            if (r.rows) take(19, 3, 32);
+            else if (conv->dtype == S3DX_F32 && blocks % 4 == 0) take(18, 4, 32);
+            else if (conv->dtype == S3DX_F32) {
+                const int nb = blocks % 3 == 0 ? 3 : blocks % 2 == 0 ? 2 : 1;
+                take(nb == 3 ? 13 : nb == 2 ? 12 : 14, nb, conv->cin % 64 == 0 ? 64 : 32);
+            }
+            return r;
+        }
     }
     if (gplan) {
         // Only the halo kernels and the three-term one read plans; other launches ignore it.
@@ -1027,7 +1046,7 @@ char *map_buffer(const s3dx_conv *conv, int64_t bytes, hipStream_t s) {
                 return nullptr;
             }
         }
-        fill_u32(static_cast<uint32_t *>(conv->fold), kFoldList, 0u, s);
+        fill_u32(static_cast<uint32_t *>(conv->fold), kFoldState, 0u, s);
     }
     return static_cast<char *>(conv->fold) + 1024;
 }
@@ -1444,25 +1463,19 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         char *fold_records = nullptr;
         if (fold) {
             const int64_t tiles = (n_in + 127) / 128;
-            const int64_t list = static_cast<int64_t>(round_up((kFoldList + tiles) * 4, 1024)) - 1024;
-            fold_records = map_buffer(conv, list + tiles * kGatherPlanRecord128, s);
+            fold_records = map_buffer(conv, tiles * kGatherPlanRecord128, s);
             if (fold_records) {
-                fold_records += list;
                 fold_state = static_cast<uint32_t *>(conv->fold);
             } else {
                 fold = 0;
+                plan = route.whole;
             }
         }
-        // Runs by 512-row tiles: the same state words, its records behind the list.
-        const int64_t row_tiles = (n_out + 511) / 512;
-        const int64_t row_list = static_cast<int64_t>(round_up((kFoldList + row_tiles) * 4, 1024)) - 1024;
+        // Runs by 512-row tiles.
         char *row_records = nullptr;
         if (route.rows) {
-            row_records = map_buffer(conv, row_list + row_tiles * kRowsRecord, s);
-            if (row_records) {
-                row_records += row_list;
-                fold_state = static_cast<uint32_t *>(conv->fold);
-            }
+            row_records = map_buffer(conv, (n_out + 511) / 512 * kRowsRecord, s);
+            if (!row_records) plan = route.whole;
         }
         if (src.pre) {
             XformArgs xa{};
@@ -1523,32 +1536,33 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
         if (route.planned) a.plan = plan.f3 ? gplan->f3_records() : gplan->d;
         if (plan.f3) a.w3 = conv->w3;
         if (fold) {
-            launch_fold_plan(kmap, n_in, fold_records, fold_state, !bf, s);
+            launch_fold_plan(kmap, n_in, fold_records, fold_state, s);
             launch_check("fold_plan");
             ConvArgs fa = a;
             fa.plan = fold_records;
-            if (!bf) {
+            if (bf) {
+                fa.w = conv->w_fold;
+                launch_conv_fold(fa, fold, s);
+                launch_check("conv_fold");
+                launch_halo_left(a, plan.nb, 1024, fold_records, kGatherPlanRecord128, fold_state, s);
+            } else {
                 fa.w3 = conv->w_fold;
-                launch_conv_f3_fold(fa, fold_state, s);
-                return;
+                launch_conv_f3_fold(fa, s);
+                launch_check("conv_f3_fold");
+                launch_splitk_left_f32(a, plan.nb, 1024, fold_records, kGatherPlanRecord128, fold_state, s);
             }
-            fa.w = conv->w_fold;
-            launch_conv_fold(fa, fold, s);
-            launch_check("conv_fold");
-            a.plan = nullptr;
-            launch_halo_listed(a, plan.nb, 16, fold_state, s);
-            launch_check("conv_halo_listed");
+            launch_check("conv_left");
             return;
         }
         if (row_records) {
-            launch_rows_plan(kmap, n_out, src.n_src, row_records, fold_state, s);
+            launch_rows_plan(kmap, n_out, src.n_src, row_records, s);
             launch_check("rows_plan");
             ConvArgs ra = a;
             ra.plan = row_records;
             launch_conv_rows(ra, s);
             launch_check("conv_rows");
-            launch_halo_listed(a, 3, 8, fold_state, s);
-            launch_check("conv_halo_listed");
+            launch_splitk_left_bf16(a, 512, row_records, kRowsRecord, static_cast<uint32_t *>(conv->fold), s);
+            launch_check("conv_left");
             return;
         }
         if (route.own) {

@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(256) f3_weights_kernel(const uint4 *w, uint4 *
 // FOLD: the folded conv over repeated parent rows (conv_fold.hip: 8 parents'
 // summed weights in place of 27 children's).  Wave s owns slot s of 64 of the
 // tile's 128 parents and 32 columns; its offsets are the slot's 8 of the parent
-// map's 27.  Tiles that the fold plan lists are left to the FP32 kernel behind.
+// map's 27.  Tiles that the fold plan marks are left to the FP32 kernel behind.
 template <int CG, int KS, bool FOLD = false>
 __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
     static_assert(FOLD ? CG == 1 && KS == 1 : 2 * CG * KS == 8, "eight waves");
@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
     const uint32_t mode = __builtin_amdgcn_readfirstlane(hdr[0]);
     const int distinct = static_cast<int>(__builtin_amdgcn_readfirstlane(hdr[1]));
     const uint32_t mask = __builtin_amdgcn_readfirstlane(hdr[2]);
-    if (FOLD && mode != 0u) return;  // a listed tile
+    if (FOLD && mode != 0u) return;  // left to the FP32 kernel behind
     // What the planes hold at a time (a pass over a chunk): the tile's distinct
     // rows; of more than they have room for, the first kF3Part, then the rest; in a
     // tile without slots (mode 1) the 128 rows that each of five offsets names.
@@ -583,44 +583,6 @@ __global__ void __launch_bounds__(256) f3_fold_weights_kernel(const float *w, ui
     }
 }
 
-// The child rows of the parent tiles that a folded FP32 run left over, with
-// FP32 matrix instructions and rows from memory: 32 rows x 32 columns a wave.
-// Usually none; no care is taken for speed.
-__global__ void __launch_bounds__(256) conv_f3_listed_kernel(ConvArgs a, uint32_t *state) {
-    const int lane = threadIdx.x & 63, half = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const int nbtot = a.cout_pad / 32;
-    const int64_t units = static_cast<int64_t>(state[kFoldCount]) * 32 * nbtot;  // 1,024 rows: 32 blocks
-    for (int64_t u = blockIdx.x * 4ll + wave; u < units; u += gridDim.x * 4ll) {
-        const int cb = static_cast<int>(u % nbtot);
-        const int64_t blk = u / nbtot;
-        const int64_t r0 = static_cast<int64_t>(state[kFoldList + blk / 32]) * 1024 + (blk % 32) * 32;
-        if (r0 >= a.n_out) continue;
-        const int64_t row = r0 + (lane & 31);
-        f32x16 acc{};
-        for (int o = 0; o < kMaxKvol; ++o) {
-            const int32_t j = row < a.n_out ? a.kmap[row * kMaxKvol + o] : -1;
-            const int32_t src = j >= 0 && j < a.n_src ? j >> a.row_shift : -1;
-            if (__builtin_amdgcn_ballot_w64(src >= 0) == 0) continue;
-            const uint4 *w = static_cast<const uint4 *>(a.w) + (static_cast<int64_t>(o) * (a.cin / 8) * nbtot + cb) * 64 + lane;
-            for (int s = 0; s < a.cin / 8; ++s)
-                acc = mfma_step<float>(
-                    gather_plain<float>(a.x, static_cast<int32_t>(a.x_bytes), src, a.cin, s * 8 + half * 4),
-                    w[static_cast<int64_t>(s) * nbtot * 64], acc);
-        }
-        const int col = cb * 32 + (lane & 31);
-        const float b = a.bias ? a.bias[col] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int64_t y = r0 + 4 * half + 8 * (r >> 2) + (r & 3);
-            float v = acc[r] + b;
-            if (a.silu) v = silu(v);
-            if (y < a.n_out) static_cast<float *>(a.y)[y * a.cout + col] = v;
-        }
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) state[kFoldBadRows] = 0u;
-}
-
 }  // namespace
 
 int64_t f3_weight_bytes(int cin, int cout_pad) { return static_cast<int64_t>(kMaxKvol) * cin * cout_pad * 6; }
@@ -641,13 +603,10 @@ void launch_f3_fold_weights(const void *w, void *out, int cin, int cout_pad, uin
                        cout_pad / 32, bad);
 }
 
-void launch_conv_f3_fold(const ConvArgs &a, uint32_t *state, hipStream_t stream) {
+void launch_conv_f3_fold(const ConvArgs &a, hipStream_t stream) {
     const unsigned tiles = static_cast<unsigned>((a.n_out / 8 + 127) / 128);
     const KernelFn fn = conv_f3_kernel<1, 1, true>;
     hipLaunchKernelGGL(fn, dim3(2 * tiles, static_cast<unsigned>(a.cout_pad / 32)), dim3(kHalo8Threads), 0, stream, a);
-    launch_check("conv_f3_fold");
-    hipLaunchKernelGGL(conv_f3_listed_kernel, dim3(std::min(tiles * 8u, 1024u)), dim3(256), 0, stream, a, state);
-    launch_check("conv_f3_listed");
 }
 
 KernelFn pick_f3(int cg) {

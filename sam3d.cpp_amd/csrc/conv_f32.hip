@@ -19,6 +19,16 @@ void launch_splitk_combine_f32(const ConvArgs &a, int64_t tiles, int groups, hip
                        dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(groups)), dim3(256), 0, stream, a);
 }
 
+void launch_splitk_left_f32(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state,
+                            hipStream_t stream) {
+    const bool wide = a.cin % 64 == 0;
+    const auto fn = nb == 4 ? launch_left<float, 4, 32, 1, 2>
+                    : nb == 3 ? (wide ? launch_left<float, 3, 64, 1, 4> : launch_left<float, 3, 32, 1, 4>)
+                    : nb == 2 ? (wide ? launch_left<float, 2, 64, 1, 4> : launch_left<float, 2, 32, 1, 4>)
+                              : (wide ? launch_left<float, 1, 64, 1, 4> : launch_left<float, 1, 32, 1, 4>);
+    fn(a, rows, records, record, state, stream);
+}
+
 KernelFn pick_linear_f32(int nbt) { return pick_linear<float>(nbt); }
 
 KernelFn pick_linear_f32_bf16_rows(int nbt) { return pick_linear<float, true>(nbt); }

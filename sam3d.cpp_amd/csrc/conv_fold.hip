@@ -27,10 +27,10 @@
 //                      one of the 8 * 27 child entries reaches the parent that
 //                      the folding assumes.  Tiles that fail it (a map that no
 //                      subdivide made), that name more rows than the halo
-//                      holds, or any when a row holds an infinity or NaN, are
-//                      listed for the general kernel.
+//                      holds (1,088), or any when a row holds an infinity or
+//                      NaN, are marked for the general kernel.
 //   conv_fold_kernel   the tiles that pass.
-//   the general halo kernel, over the listed tiles (conv_halo.hip).
+//   the general halo kernel, over the marked tiles (conv_halo.hip).
 #include "halo_tile.hpp"
 
 namespace s3dx {
@@ -134,7 +134,7 @@ struct FoldSlice {
 };
 
 __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const int32_t *kmap, int64_t n_parents,
-                                                                         char *plan, uint32_t *state, int most) {
+                                                                         char *plan, const uint32_t *state) {
     // A parent's 8 * 27 child entries are 54 16-byte pieces; 864 of the threads
     // take the pieces of 16 parents a pass, each thread the same piece of
     // every parent, so that what its four entries are (the parent offset they
@@ -198,11 +198,8 @@ __global__ void __launch_bounds__(kPlanBuild128Threads) fold_plan_kernel(const i
     const TileDedupe dd = plan_tile<4, NTH>(FoldSlice{parents}, n_parents, n_parents, 0, plan);
     // (plan_tile's barriers order the writes of `wrong` before this read, and
     // thread 0 wrote the record's header)
-    if (tid == 0 && (wrong != 0u || dd.global_a || dd.distinct > static_cast<uint32_t>(most))) {
+    if (tid == 0 && (wrong != 0u || dd.global_a))
         *reinterpret_cast<uint32_t *>(plan + static_cast<int64_t>(tile) * kGatherPlanRecord128) = kFoldGeneral;
-        const uint32_t at = atomicAdd(state + kFoldCount, 1u);
-        state[kFoldList + at] = static_cast<uint32_t>(tile);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -265,9 +262,13 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
     const uint32_t *hdr = reinterpret_cast<const uint32_t *>(rec);
     if (__builtin_amdgcn_readfirstlane(hdr[0]) != 0u) return;  // the general kernel's
     const int distinct = static_cast<int>(__builtin_amdgcn_readfirstlane(hdr[1]));
-    if (tid < 2 * (kHRowBytes / 16))  // each buffer's zero row
-        reinterpret_cast<uint4 *>(halo + ((tid / (kHRowBytes / 16)) * kH8BufRows + kH8Double) * kHRowBytes)[tid % (kHRowBytes / 16)] =
-            make_uint4(0, 0, 0, 0);
+    // Tiles of more rows than two buffers hold (no thin shell's: of a solid bar of
+    // 24 x 24 x 60 most) take one, whose copy nothing hides: about 5% of a chunk.
+    const bool single = distinct > kH8Double;
+    if (tid < 2 * (kHRowBytes / 16)) {  // each buffer's zero row, or the one's
+        const int zero = single ? kH8Single : (tid / (kHRowBytes / 16)) * kH8BufRows + kH8Double;
+        reinterpret_cast<uint4 *>(halo + zero * kHRowBytes)[tid % (kHRowBytes / 16)] = make_uint4(0, 0, 0, 0);
+    }
 
     const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.x), static_cast<short>(0),
                                                           static_cast<int32_t>(a.x_bytes), 0x00020000);
@@ -285,7 +286,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
         const int p = (ln & 7) ^ halo_swizzle(sl);
         // (24 bits: rows * 128 bytes at least are below 2 GiB; the top bit
         // puts a slot past the last row out of range: zeros)
-        const uint32_t off = (__umul24(rows[min(sl, kH8Double)], 2u * static_cast<uint32_t>(a.cin)) + p * 16u) |
+        const uint32_t off = (__umul24(rows[min(sl, kH8Single - 1)], 2u * static_cast<uint32_t>(a.cin)) + p * 16u) |
                              (sl < distinct ? 0u : 0x80000000u);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (__attribute__((address_space(3))) void *)(dst + g * 1024), 16,
                                                  static_cast<int32_t>(off), c * kHRowBytes, 0, 0);
@@ -312,8 +313,14 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
     const int bx = (wave >> 2) & 1, by = (wave >> 1) & 1, bz = wave & 1;
     const int ox = bx ? 18 : 0, oy = by ? 6 : 0, oz = bz ? 2 : 0;
 
+    constexpr int kPiecesSingle = (kH8Single + 63) / 64;
+    if (single) {
+#pragma nounroll
+        for (int j = 0; j < kPiecesSingle; ++j) piece(j, 0, halo, slot_row);
+    } else {
 #pragma unroll
-    for (int j = 0; j < kPieces; ++j) piece(j, 0, halo, slot_row);
+        for (int j = 0; j < kPieces; ++j) piece(j, 0, halo, slot_row);
+    }
 #pragma unroll
     for (int k = 0; k < RB; ++k) {
 #pragma unroll
@@ -324,7 +331,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
     // weights requested over the last steps.
     auto chunk = [&](int c, const char *__restrict__ buf, char *__restrict__ nxt, const uint32_t *__restrict__ tbl,
                      const uint32_t *__restrict__ rows) __attribute__((always_inline)) {
-        const bool last = c + 1 == chunks;
+        const bool last = c + 1 == chunks, copy = !last && !single;
         int32_t wb = w_first + c * kFoldSlots * slot_bytes + RB * step_bytes;  // the next step to request
         // the steps past this chunk's are the next chunk's first (the last
         // chunk reads its own first ones again: unused)
@@ -357,7 +364,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
             // the next group's rows, once this group's last fragments are read
             if constexpr (last_term && k == 3 && more) load_ix(std::integral_constant<int, m + 1 < 8 ? m + 1 : 0>{});
             if constexpr (t % 2 == 0 && t / 2 < kPieces)
-                if (!last) piece(t / 2, c + 1, nxt, rows);
+                if (copy) piece(t / 2, c + 1, nxt, rows);
             // Row blocks 0 and 1 over all column blocks, then 2 and 3: an A
             // fragment is refilled half a step before its next use, a weight
             // fragment a step and a third (fenced: each takes the registers
@@ -383,9 +390,17 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_fold_kernel(ConvArgs a)
     for (int c = 0; c < chunks; ++c) {
         // chunk c's pieces precede the RB weight sets in flight; after the
         // barrier no wave reads the buffer of chunk c - 1
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(RB * NBW));
+        if (single && c > 0) {
+            __syncthreads();
+#pragma nounroll
+            for (int j = 0; j < kPiecesSingle; ++j) piece(j, c, halo, slot_row);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        } else {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(RB * NBW));
+        }
         __syncthreads();
-        char *cur = halo + (c & 1) * (kH8BufRows * kHRowBytes), *nxt = halo + ((c + 1) & 1) * (kH8BufRows * kHRowBytes);
+        char *cur = single ? halo : halo + (c & 1) * (kH8BufRows * kHRowBytes);
+        char *nxt = halo + ((c + 1) & 1) * (kH8BufRows * kHRowBytes);
         chunk(c, cur, nxt, table, slot_row);
     }
 
@@ -470,10 +485,9 @@ void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t
                        bad);
 }
 
-void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, bool f32, hipStream_t stream) {
+void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, const uint32_t *state, hipStream_t stream) {
     hipLaunchKernelGGL(fold_plan_kernel, dim3(static_cast<unsigned>((n_parents + 127) / 128)),
-                       dim3(kPlanBuild128Threads), 0, stream, kmap, n_parents, static_cast<char *>(plan), state,
-                       f32 ? kH8Single : kH8Double);
+                       dim3(kPlanBuild128Threads), 0, stream, kmap, n_parents, static_cast<char *>(plan), state);
 }
 
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream) {

@@ -36,8 +36,9 @@ namespace {
 
 // NB 32-column blocks per tile: 4 (128 columns), or 3 (96 columns: wave w < 3
 // owns column block w in the reduction, wave 3 only hands its partials over).
-template <int MB, bool PLAN, int NB>
-__device__ __forceinline__ void halo_body(const ConvArgs &a, const int tile, const int nb0) {
+// LEFT: the tiles that a folded run left over (is_left).
+template <int MB, bool PLAN, int NB = 4, bool LEFT = false>
+__global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_halo_kernel(ConvArgs a) {
     static_assert(NB == 4 || NB == 3, "128- or 96-column tiles");
     using SM = HaloSmem<MB>;
     constexpr int ROWS = SM::ROWS, CAP = SM::CAP, RPH = SM::RPH;
@@ -51,6 +52,10 @@ __device__ __forceinline__ void halo_body(const ConvArgs &a, const int tile, con
     int32_t *misc = reinterpret_cast<int32_t *>(smem + SM::MISC_OFF);  // [0] lo, [1] hi, [2] mask, [4..7] scan
     int32_t *table32 = reinterpret_cast<int32_t *>(PLAN ? rec + kPlanHeader : smem);  // global-gather mode
 
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    if constexpr (LEFT)
+        if (!is_left(a.left, tile)) return;
+    const int nb0 = blockIdx.y * NB;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5;
@@ -349,27 +354,6 @@ __device__ __forceinline__ void halo_body(const ConvArgs &a, const int tile, con
     load_residual<TPR, ROWS>(a, m0, nb0, tile_rows, tid, res);
     __syncthreads();
     finish_rows<TPR, ROWS, SM::STG_LD>(a, stg, part, m0, nb0, tile_rows, tid, res);
-}
-
-template <int MB, bool PLAN, int NB = 4>
-__global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_halo_kernel(ConvArgs a) {
-    halo_body<MB, PLAN, NB>(a, xcd_tile(blockIdx.x, gridDim.x), blockIdx.y * NB);
-}
-
-// The 64-row tiles of the larger tiles (per of them each) that a folded run,
-// or one by 512-row tiles, left over, by however many workgroups there are;
-// usually none.
-template <int NB>
-__global__ void __launch_bounds__(256, 1) conv_halo_listed_kernel(ConvArgs a, int per, uint32_t *state) {
-    const int64_t total = static_cast<int64_t>(state[kFoldCount]) * per;
-    const int64_t tiles = (a.n_out + 63) / 64;
-    for (int64_t i = blockIdx.x; i < total; i += gridDim.x) {
-        const int64_t tile = static_cast<int64_t>(state[kFoldList + i / per]) * per + i % per;
-        if (tile >= tiles) continue;
-        __syncthreads();  // the previous tile is done with LDS
-        halo_body<2, false, NB>(a, static_cast<int>(tile), blockIdx.y * NB);
-    }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) state[kFoldBadRows] = 0u;
 }
 
 // 128-row x 128-column tiles read through 128-row gather-plan records: one
@@ -1118,11 +1102,11 @@ KernelFn pick_halo_bf16(int rows, int nb) {
     return rows == 128 ? conv_halo_kernel<4, false> : rows == 64 ? conv_halo_kernel<2, false> : nullptr;
 }
 
-void launch_halo_listed(const ConvArgs &a, int nb, int per, uint32_t *state, hipStream_t stream) {
-    const unsigned tiles = static_cast<unsigned>(std::min<int64_t>((a.n_out + 63) / 64, 512));
-    const dim3 grid(tiles, static_cast<unsigned>(a.cout_pad / 32 / nb));
-    if (nb == 3) hipLaunchKernelGGL(conv_halo_listed_kernel<3>, grid, dim3(256), 0, stream, a, per, state);
-    else hipLaunchKernelGGL(conv_halo_listed_kernel<4>, grid, dim3(256), 0, stream, a, per, state);
+void launch_halo_left(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state, hipStream_t stream) {
+    a.left = LeftTiles{static_cast<const char *>(records), state, record, rows / 64};
+    const KernelFn fn = nb == 3 ? conv_halo_kernel<2, false, 3, true> : conv_halo_kernel<2, false, 4, true>;
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((a.n_out + 63) / 64), static_cast<unsigned>(a.cout_pad / 32 / nb)), dim3(256), 0,
+                       stream, a);
 }
 
 KernelFn pick_halo8_stream_k() { return conv_halo8_sk_kernel; }

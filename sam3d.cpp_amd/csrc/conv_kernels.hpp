@@ -9,6 +9,19 @@
 
 namespace s3dx {
 
+// The tiles that a plan kernel leaves to a general one: its records' first word is
+// kFoldGeneral.  The general kernel's launch is over all of its own row tiles (`per`
+// of them in a record's tile), and workgroups whose tile is done return: 1.2 ns each,
+// 33 us of 1,000 at 1.81M rows, where usually none is left.  (Where all are -- rows in
+// no order -- anything that shares them out among fewer workgroups costs more:
+// four tiles a workgroup 4%, lists dealt out in turn 6%, queues of one atomic a tile
+// 12-33%.)
+struct LeftTiles {
+    const char *records;
+    uint32_t *state;
+    int32_t record, per;
+};
+
 struct ConvArgs {
     const void *x;
     int64_t x_bytes;  // bytes addressable at x
@@ -41,6 +54,7 @@ struct ConvArgs {
     int32_t sk_wgs;
     int64_t sk_units;
     float *sk_partial;
+    LeftTiles left;  // the general kernels' launches over left tiles
 };
 
 using KernelFn = void (*)(ConvArgs);
@@ -121,28 +135,31 @@ KernelFn pick_f3(int cg);
 // run with the FP32 pass over the listed tiles behind it.
 int64_t f3_fold_weight_bytes(int cin, int cout_pad);
 void launch_f3_fold_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
-void launch_conv_f3_fold(const ConvArgs &a, uint32_t *state, hipStream_t stream);
-// Folded convs over repeated parent rows (conv_fold.hip).  `state`: the words
-// below, then the list (one word per 128 parents); the count is cleared before
-// each run's plan, the flag by the listed pass that ends a run.
-constexpr int kFoldCount = 0;    // parent tiles left to the general kernel
-constexpr int kFoldBadRows = 1;  // a source row holds an infinity or NaN
-constexpr int kFoldList = 4;     // the tiles counted
-constexpr uint32_t kFoldGeneral = 2;  // record mode of those tiles
+void launch_conv_f3_fold(const ConvArgs &a, hipStream_t stream);
+// Folded convs over repeated parent rows (conv_fold.hip), and the 512-row tiles of
+// conv_rows.hip.  `state`: the flag below, raised by the row pass and cleared by
+// the general kernel's launch that ends a run.
+constexpr int kFoldBadRows = 0;       // a source row holds an infinity or NaN
+constexpr int kFoldState = 16;        // words
+constexpr uint32_t kFoldGeneral = 2;  // record mode of the tiles left to a general kernel
 int64_t fold_weight_bytes(int cin, int blocks);
 int fold_blocks(int cin, int blocks, int general_nb, int64_t n_parents, int64_t cus);
 // *bad: raised when a folded weight is no finite number.
 void launch_fold_weights(const void *w, void *out, int cin, int blocks, uint32_t *bad, hipStream_t stream);
-void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, uint32_t *state, bool f32, hipStream_t stream);
+void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, const uint32_t *state, hipStream_t stream);
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
-// The general kernel (64-row tiles, nb column blocks) over the listed tiles of
-// `per` * 64 rows.
-void launch_halo_listed(const ConvArgs &a, int nb, int per, uint32_t *state, hipStream_t stream);
+// The general kernels over the tiles of `rows` rows that the records (of `record`
+// bytes) leave over: the 64-row halo kernel of nb column blocks, and split-K
+// kernels (BF16: tiling 19 on 32-channel chunks; FP32: tiling 18, 13, 12 or 14 for
+// nb 4, 3, 2 or 1).
+void launch_halo_left(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state, hipStream_t stream);
+void launch_splitk_left_bf16(ConvArgs a, int rows, const void *records, int record, uint32_t *state, hipStream_t stream);
+void launch_splitk_left_f32(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state,
+                            hipStream_t stream);
 // BF16 convs over many rows, 96 columns a workgroup (conv_rows.hip): a record
-// per 512 rows, and the state words above for the tiles left to the general
-// kernel.
+// per 512 rows.
 constexpr int kRowsRecord = 34816;
-void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, uint32_t *state, hipStream_t stream);
+void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, hipStream_t stream);
 void launch_conv_rows(const ConvArgs &a, hipStream_t stream);
 // The FP32 1x1-layer kernel reading BF16 rows, else nullptr.
 KernelFn pick_linear_f32_bf16_rows(int nbt);
@@ -167,6 +184,13 @@ template <>
 struct Frag<float> {
     static constexpr int E = 4;
 };
+
+// Whether a general kernel's row tile was left to it.
+__device__ __forceinline__ bool is_left(const LeftTiles &l, int tile) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) l.state[kFoldBadRows] = 0u;
+    const uint32_t mode = *reinterpret_cast<const uint32_t *>(l.records + static_cast<int64_t>(tile / l.per) * l.record);
+    return __builtin_amdgcn_readfirstlane(mode) == kFoldGeneral;
+}
 
 // One 16-byte fragment of source row j (already shifted), channels c0 ..
 // c0+E, with 64-bit addressing; a zero fragment when j < 0.
@@ -909,8 +933,12 @@ __device__ __forceinline__ int sk_run_of(int64_t u, int64_t units, int32_t runs)
 // tile, task) units, tasks counted over all kvol offsets of a tile, as the
 // 8-wave halo kernel's (equal runs, whole tiles finished here, parts of a
 // tile left as FP32 tiles in the run's two slots for splitk_combine_kernel).
-template <class T, int NB, int KC, int XF, int SUB, int MB, bool SK>
+//
+// kLeftTiles (conv_splitk_left_kernel): the tiles that a plan kernel left over.
+enum SplitMode { kWholeTiles, kStreamK, kLeftTiles };
+template <class T, int NB, int KC, int XF, int SUB, int MB, SplitMode MODE>
 __device__ __forceinline__ void splitk_body(const ConvArgs &a) {
+    constexpr bool SK = MODE == kStreamK;
     static_assert(!SK || SUB == 1, "stream-K runs walk single-chunk tasks");
     using SM = SplitSmem<T, NB, KC, MB>;
     constexpr int RPH = SM::RPH;
@@ -1454,8 +1482,11 @@ __device__ __forceinline__ void splitk_body(const ConvArgs &a) {
         finish_rows<SM::TPR, BM, SM::STG_LD>(a, stg, part, m0, nb0, tile_rows, tid, res);
     }
     };
-    if constexpr (!SK) {
+    if constexpr (MODE == kWholeTiles) {
         piece(xcd_tile(blockIdx.x, gridDim.x), blockIdx.y * NB, 0, INT32_MAX, nullptr);
+    } else if constexpr (MODE == kLeftTiles) {
+        const int tile = xcd_tile(blockIdx.x, gridDim.x);
+        if (is_left(a.left, tile)) piece(tile, blockIdx.y * NB, 0, INT32_MAX, nullptr);
     } else {
         const int64_t tiles = (a.n_out + BM - 1) / BM;
         const int64_t ntf = static_cast<int64_t>(a.kvol) * chunks_all;  // nominal tasks per tile
@@ -1479,11 +1510,22 @@ __device__ __forceinline__ void splitk_body(const ConvArgs &a) {
 
 template <class T, int NB, int KC, int XF, int SUB, int MB>
 __global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_splitk_kernel(ConvArgs a) {
-    splitk_body<T, NB, KC, XF, SUB, MB, false>(a);
+    splitk_body<T, NB, KC, XF, SUB, MB, kWholeTiles>(a);
 }
 template <class T, int NB, int KC, int XF, int SUB, int MB>
 __global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_splitk_sk_kernel(ConvArgs a) {
-    splitk_body<T, NB, KC, XF, SUB, MB, true>(a);
+    splitk_body<T, NB, KC, XF, SUB, MB, kStreamK>(a);
+}
+template <class T, int NB, int KC, int SUB, int MB>
+__global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_splitk_left_kernel(ConvArgs a) {
+    splitk_body<T, NB, KC, 0, SUB, MB, kLeftTiles>(a);
+}
+template <class T, int NB, int KC, int SUB, int MB>
+void launch_left(ConvArgs &a, int rows, const void *records, int record, uint32_t *state, hipStream_t stream) {
+    a.left = LeftTiles{static_cast<const char *>(records), state, record, rows / (32 * MB)};
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_splitk_left_kernel<T, NB, KC, SUB, MB>),
+                       dim3(static_cast<unsigned>((a.n_out + 32 * MB - 1) / (32 * MB)), static_cast<unsigned>(a.cout_pad / 32 / NB)),
+                       dim3(256), 0, stream, a);
 }
 
 // The tiles that a split-K kernel's stream-K runs left in parts: the pieces'

@@ -25,7 +25,7 @@
 //                      27 * 512 map entries and each entry's slot among them
 //   conv_rows_kernel   the tiles with all 27 offsets (any 2x2x2 block of
 //                      children has them) and at most 1,535 distinct rows
-//   the 64-row halo kernel, over the other tiles (conv_halo.hip)
+//   the 64-row split-K kernel, over the other tiles (conv_kernels.hpp)
 #include "halo_tile.hpp"
 
 namespace s3dx {
@@ -44,9 +44,8 @@ static_assert(kRowsRecord % 1024 == 0, "whole KiB");
 // Table entries: the offset of piece 0 in 16-byte units.
 __device__ __forceinline__ uint32_t rows_entry(uint32_t s) { return s * 4 + ((s >> 1) & 3); }
 
-// One workgroup per tile.  state: the listed tiles (kFoldCount, kFoldList).
-__global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, int64_t n_out, int64_t n_src, char *plan,
-                                                         uint32_t *state) {
+// One workgroup per tile.
+__global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, int64_t n_out, int64_t n_src, char *plan) {
     constexpr int NTH = 1024, WORDS = 4096;  // a bitmap over 131,072 rows
     constexpr int V4 = kRowsTile * kMaxKvol / 4, Q = (V4 + NTH - 1) / NTH;
     __shared__ __align__(16) uint16_t table[kRowsTile * kMaxKvol];
@@ -103,9 +102,9 @@ __global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, in
     }
     const int rlo = misc[0], rhi = misc[1];
     const int64_t span = rhi >= rlo ? static_cast<int64_t>(rhi) - rlo + 1 : 0;
-    bool listed = misc[2] != (1 << kMaxKvol) - 1 || span > static_cast<int64_t>(WORDS) * 32;
+    bool left = misc[2] != (1 << kMaxKvol) - 1 || span > static_cast<int64_t>(WORDS) * 32;
     uint32_t distinct = 0;
-    if (!listed) {
+    if (!left) {
 #pragma unroll
         for (int q = 0; q < Q; ++q)
 #pragma unroll
@@ -133,15 +132,12 @@ __global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, in
             prefix[tid * WPT + k] = run;
             run += cnt[k];
         }
-        listed = distinct >= static_cast<uint32_t>(kRowsCap);
+        left = distinct >= static_cast<uint32_t>(kRowsCap);
         __syncthreads();
     }
     char *rec = plan + static_cast<int64_t>(tile) * kRowsRecord;
-    if (listed) {
-        if (tid == 0) {
-            *reinterpret_cast<uint4 *>(rec) = make_uint4(kFoldGeneral, 0u, 0u, 0u);
-            state[kFoldList + atomicAdd(state + kFoldCount, 1u)] = static_cast<uint32_t>(tile);
-        }
+    if (left) {
+        if (tid == 0) *reinterpret_cast<uint4 *>(rec) = make_uint4(kFoldGeneral, 0u, 0u, 0u);
         return;
     }
 #pragma unroll
@@ -184,7 +180,7 @@ __global__ void __launch_bounds__(256, 1) conv_rows_kernel(ConvArgs a) {
     const int chunks = a.cin / kChunk, ksteps = a.cin / 16;
     const char *rec = static_cast<const char *>(a.plan) + static_cast<int64_t>(tile) * kRowsRecord;
     const uint4 hdr = *reinterpret_cast<const uint4 *>(rec);
-    if (__builtin_amdgcn_readfirstlane(hdr.x) != 0u) return;  // a listed tile
+    if (__builtin_amdgcn_readfirstlane(hdr.x) != 0u) return;  // left to the general kernel
     const int distinct = static_cast<int>(__builtin_amdgcn_readfirstlane(hdr.y));
 
     const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.x), static_cast<short>(0),
@@ -347,9 +343,9 @@ __global__ void __launch_bounds__(256, 1) conv_rows_kernel(ConvArgs a) {
 
 }  // namespace
 
-void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, uint32_t *state, hipStream_t stream) {
+void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, hipStream_t stream) {
     hipLaunchKernelGGL(rows_plan_kernel, dim3(static_cast<unsigned>((n_out + kRowsTile - 1) / kRowsTile)), dim3(1024), 0,
-                       stream, kmap, n_out, n_src, static_cast<char *>(plan), state);
+                       stream, kmap, n_out, n_src, static_cast<char *>(plan));
 }
 
 void launch_conv_rows(const ConvArgs &a, hipStream_t stream) {

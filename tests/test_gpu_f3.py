@@ -64,6 +64,7 @@ CASES = {
     "solid_bar": (lambda W: _box(16, 24, 60), 64, 128, False, 128),                            # up to 750: two parts
     "solid_bar_two_k": (lambda W: _box(12, 15, 60), 64, 192, False, 64),
     "solid_bar_four_k": (lambda W: _box(12, 24, 60), 64, 96, False, 32),
+    "shuffled_whole_row": (lambda W: _shuffled(W.shells_union(0)[:12801]), 128, 128, True, 128),
     "shuffled_two_k": (lambda W: _shuffled(W.shells_union(0)[:9000]), 64, 192, False, 64),
     "shuffled_four_k": (lambda W: _shuffled(W.shells_union(0)[:9000]), 64, 96, False, 32),
     "shuffled": (lambda W: _shuffled(W.shells_union(0)[:12000]), 64, 128, False, None),        # the plan's global tiles

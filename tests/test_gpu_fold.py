@@ -255,3 +255,44 @@ def test_refused_plan_leaves_nothing_behind(s3dx, W):
     with pytest.raises(s3dx.S3dxError):
         conv.run(s3dx.DeviceArray.from_host(W.f32_to_bf16_bits(xi)), p, kd, 8 * p, y, s3dx.BF16, plan=gp)
     assert np.array_equal(_run(s3dx, W, conv, x, kmap, cout), first)
+
+
+def _box(x, y, z):
+    g = np.stack(np.meshgrid(np.arange(x), np.arange(y), np.arange(z), indexing="ij"), -1).reshape(-1, 3) + 2
+    return np.ascontiguousarray(np.concatenate([np.zeros((len(g), 1), np.int64), g], 1).astype(np.int32))
+
+
+def _against_both(s3dx, O, W, monkeypatch, parents, cin, cout):
+    p = parents.shape[0]
+    conv, kmap, x, w, b, scale, shift = _setup(s3dx, W, parents, cin, cout)
+    assert " fold " in conv.plan(p, 8 * p)
+    got = _run(s3dx, W, conv, x, kmap, cout)
+    assert np.array_equal(got, _run(s3dx, W, conv, x, kmap, cout)), "two runs differ"
+    want = _general(s3dx, W, monkeypatch, conv, x, kmap, cout)
+    g, v = (W.bf16_bits_to_f32(t).reshape(t.shape) for t in (got, want))
+    assert np.linalg.norm(g - v) < 2.0 ** -11 * np.linalg.norm(v)
+    rows = np.unique(np.concatenate([np.random.default_rng(1).choice(8 * p, 1500, replace=False), [0, 8 * p - 1]]))
+    a = W.round_bf16(O.silu((x * scale + shift).astype(np.float32)))
+    km = np.where(kmap[rows] >= 0, kmap[rows] >> 3, -1).astype(np.int32)
+    check_rel(g[rows], O.conv(a, km, p, W.round_bf16(w), 1, cout, b), 1e-2, "oracle")
+    return np.mean((got == want).reshape(-1, 1024 * cout).all(1)) if p % 128 == 0 else None
+
+
+@pytest.mark.parametrize("shape,cin,cout", [((16, 24, 60), 192, 96), ((16, 24, 64), 128, 128), ((7, 24, 64), 256, 192)])
+def test_solid_sets(s3dx, O, W, monkeypatch, shape, cin, cout):
+    # Solid sets name more parents in a tile (up to 768) than two halo buffers hold
+    # (559): those tiles are folded over one buffer.
+    parents = _box(*shape)
+    km = O.kmap_subm3(parents, parents.shape[0])
+    most = [len(np.unique(t[t < parents.shape[0]])) for t in np.split(km, range(128, len(km), 128))]
+    print(f"{shape}: {max(most)} parents, {np.mean(np.array(most) > 559):.2f} of the tiles above 559", flush=True)
+    assert max(most) > 700 and np.mean(np.array(most) > 559) > 0.5
+    same = _against_both(s3dx, O, W, monkeypatch, parents, cin, cout)
+    assert same is None or same < 0.05  # (nearly every tile is folded: none of the general kernel's bits)
+
+
+def test_rows_in_no_order(s3dx, O, W, monkeypatch):
+    # Parents in no order: every tile goes to the general kernel.
+    c = W.shells_union(0)[:12800]
+    same = _against_both(s3dx, O, W, monkeypatch, np.ascontiguousarray(c[np.random.default_rng(4).permutation(len(c))]), 192, 96)
+    assert same == 1.0

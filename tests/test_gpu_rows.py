@@ -3,7 +3,7 @@ decoder's last conv.  Against the split-K kernel (S3DX_CONV_TILING=19): both
 accumulate in FP32 and round once to BF16, in different orders, so the outputs
 differ by one BF16 step here and there (rel-L2 far below 2^-9).  Tiles without
 all 27 offsets, of more rows than the LDS holds, or of rows further apart than
-the plan's bitmap run the 64-row halo kernel.
+the plan's bitmap run the 64-row split-K kernel: the same bits.
 """
 import numpy as np
 import pytest
@@ -22,7 +22,7 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
     kmap = kd.download()
     whole = kmap.copy()
     kmap[512 * 3:512 * 4, 5] = -1                    # an offset that no row of the tile has
-    kmap[512 * 7 + 100, 20] = n - 1                  # a row far away
+    kmap[100, 20] = n - 1                            # a row far away: 131,367 rows from the tile's first
     rng = np.random.default_rng(1)
     kmap[512 * 9:512 * 10] = rng.integers(-1, 16000, (512, 27), dtype=np.int32)  # too many rows
     kmap[512 * 256 + 3] = -1
@@ -48,7 +48,7 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
 
     a = W.round_bf16(O.silu((x * scale + shift).astype(np.float32)))
     rows = np.unique(np.concatenate([np.sort(rng.choice(n, 1200, replace=False)), np.arange(512 * 3, 512 * 3 + 40),
-                                     [512 * 7 + 100, 512 * 9 + 5, 512 * 256 + 3, n - 1]]))
+                                     [100, 512 * 9 + 5, 512 * 256 + 3, n - 1]]))
     for name, m in (("subdivide's map", whole), ("with other tiles", kmap)):
         got = run(m)
         assert np.array_equal(got, run(m)), "two runs differ"
@@ -59,6 +59,9 @@ def test_rows_kernel(s3dx, O, W, monkeypatch, cin, cout, residual, silu):
         rel = float(np.linalg.norm(g - v) / np.linalg.norm(v))
         print(f"{cin}->{cout} {name}: rel-L2 against split-K {rel:.2e}", flush=True)
         assert 0.0 < rel < 2.0 ** -11
+        if m is kmap:
+            for t in (0, 3, 9):  # the listed tiles
+                assert np.array_equal(got[512 * t:512 * t + 512], want[512 * t:512 * t + 512]), t
         ref = O.conv(a, m[rows], n, W.round_bf16(w), 1, cout, b)
         ref = O.silu(ref) if silu else ref
         check_rel(g[rows], ref + (res[rows >> 3] if residual else 0.0), 1e-2, "oracle")
