@@ -834,7 +834,8 @@ void apply_gather_plan(LaunchPlan &p, const s3dx_conv *conv, const s3dx_gather_p
 
 // A run, over no plan that it could read, of an FP32 layer that has buffers of its
 // own (input transforms): as three BF16 terms, with the map's 128-row records built in
-// the run where that pays (about 10 us).
+// the run where that pays (about 10 us: 96 -> 96 on 6,400 rows 45.5 us against 44.1
+// by FP32 instructions, 8,000 47.3 / 47.8, 8,800 49.2 / 58.4).
 bool f3_own_plan(const s3dx_conv *conv, LaunchPlan &p, const Source &src, int64_t n_out) {
     if (!src.pre || conv->dtype != S3DX_F32 || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
         (n_out + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31) || n_out < 8192)
@@ -909,8 +910,8 @@ int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src
 // Whether a run goes by 512-row tiles (conv_rows.hip): a BF16 layer
 // with an input affine (so with buffers of its own) that no halo kernel suits
 // (Cin 32 above a multiple of 64), 96-column groups, BF16 output and no
-// LayerNorm, over at least as many tiles as CUs (96 -> 96 on 256,000 rows: 176
-// against 225 us; below, the 64-row tiles fill the GPU better).
+// LayerNorm, over at least as many tiles as CUs (96 -> 96 on 256 tiles 86 us
+// against 104 by 64-row split-K tiles, on 100 tiles 67 against 61).
 bool rows_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_out, int32_t y_dtype) {
     return p.mfma && !p.linear && p.tl && p.tl->id != 20 && p.tl->id != 21 && !p.xf && conv->kvol == kMaxKvol &&
            conv->dtype == S3DX_BF16 && conv->pre_scale && src.shift == 0 && !conv->ln && y_dtype == S3DX_BF16 &&
@@ -991,6 +992,18 @@ Route route_of(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const Sourc
         r.own = f3_own_plan(conv, r.p, src, n_out);
     }
     return r;
+}
+
+// How many of the n_out rows' 512-row tiles such a run takes: all, or the whole
+// passes over the CUs (one workgroup each) where fewer than 3/8 of the CUs would
+// work in the last one; the split-K kernel then takes the rest (96 -> 96: a pass
+// is 37 us and 0.09 a tile, split-K 0.37 a tile.  All by 512 rows / all by split-K /
+// shared, us: 257 tiles 128 / 113-121 / 110-114, 300 129 / 126-134 / 119, 340 130 /
+// 136-148 / 137, 513 189 / 202-218 / 176-185).
+int64_t rows_tiles(const s3dx_conv *conv, int64_t n_out) {
+    const int64_t tiles = (n_out + 511) / 512, groups = conv->cout / 96, cus = device_cus();
+    const int64_t whole = tiles * groups / cus * cus / groups;
+    return 8 * (tiles - whole) * groups < 3 * cus ? whole : tiles;
 }
 
 float *upload_f32(const float *host, size_t count) {
@@ -1402,7 +1415,7 @@ void describe_launch(const s3dx_conv *conv, const s3dx_gather_plan *gplan, int64
                           static_cast<long long>((n_in + 127) / 128 * (conv->dtype == S3DX_F32 ? 2 : 1)),
                           conv->cout_pad / 32 / r.fold);
         else if (r.rows)
-            std::snprintf(most, sizeof(most), "rows=512 cols=96 grid=%lldx%d else ", static_cast<long long>((n_out + 511) / 512),
+            std::snprintf(most, sizeof(most), "rows=512 cols=96 grid=%lldx%d else ", static_cast<long long>(rows_tiles(conv, n_out)),
                           conv->cout / 96);
         std::snprintf(plan, plan_capacity, "%s%s%s%s%s%s", bf16_rows ? (r.widen ? "in=bf16 pre=widen " : "in=bf16 ") : "",
                       src.pre ? (src.children ? "pre=children " : "pre=rows ") : "", src.shift ? "parent-rows " : "",
@@ -1555,13 +1568,14 @@ void conv_run_impl(const s3dx_conv *conv, const s3dx_gather_plan *gplan, const v
             return;
         }
         if (row_records) {
-            launch_rows_plan(kmap, n_out, src.n_src, row_records, s);
+            const int64_t tiles = rows_tiles(conv, n_out);
+            launch_rows_plan(kmap, n_out, src.n_src, tiles, row_records, s);
             launch_check("rows_plan");
             ConvArgs ra = a;
             ra.plan = row_records;
-            launch_conv_rows(ra, s);
+            launch_conv_rows(ra, tiles, s);
             launch_check("conv_rows");
-            launch_splitk_left_bf16(a, 512, row_records, kRowsRecord, static_cast<uint32_t *>(conv->fold), s);
+            launch_splitk_left_bf16(a, 512, tiles, row_records, kRowsRecord, static_cast<uint32_t *>(conv->fold), s);
             launch_check("conv_left");
             return;
         }

@@ -13,8 +13,9 @@ KernelFn pick_mfma_bf16(int id, int kc, bool xf) {
     }
 }
 
-void launch_splitk_left_bf16(ConvArgs a, int rows, const void *records, int record, uint32_t *state, hipStream_t stream) {
-    launch_left<uint16_t, 3, 128, 4, 2>(a, rows, records, record, state, stream);
+void launch_splitk_left_bf16(ConvArgs a, int rows, int64_t tiles, const void *records, int record, uint32_t *state,
+                             hipStream_t stream) {
+    launch_left<uint16_t, 3, 128, 4, 2>(a, rows, tiles, records, record, state, stream);
 }
 
 KernelFn pick_linear_bf16(int nbt) { return pick_linear<uint16_t>(nbt); }

@@ -26,7 +26,7 @@ void launch_splitk_left_f32(ConvArgs a, int nb, int rows, const void *records, i
                     : nb == 3 ? (wide ? launch_left<float, 3, 64, 1, 4> : launch_left<float, 3, 32, 1, 4>)
                     : nb == 2 ? (wide ? launch_left<float, 2, 64, 1, 4> : launch_left<float, 2, 32, 1, 4>)
                               : (wide ? launch_left<float, 1, 64, 1, 4> : launch_left<float, 1, 32, 1, 4>);
-    fn(a, rows, records, record, state, stream);
+    fn(a, rows, (a.n_out + rows - 1) / rows, records, record, state, stream);
 }
 
 KernelFn pick_linear_f32(int nbt) { return pick_linear<float>(nbt); }

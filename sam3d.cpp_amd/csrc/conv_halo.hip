@@ -1103,10 +1103,10 @@ KernelFn pick_halo_bf16(int rows, int nb) {
 }
 
 void launch_halo_left(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state, hipStream_t stream) {
-    a.left = LeftTiles{static_cast<const char *>(records), state, record, rows / 64};
+    const int64_t row_tiles = (a.n_out + 63) / 64;
+    a.left = LeftTiles{static_cast<const char *>(records), state, record, rows / 64, static_cast<int32_t>(row_tiles)};
     const KernelFn fn = nb == 3 ? conv_halo_kernel<2, false, 3, true> : conv_halo_kernel<2, false, 4, true>;
-    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((a.n_out + 63) / 64), static_cast<unsigned>(a.cout_pad / 32 / nb)), dim3(256), 0,
-                       stream, a);
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(row_tiles), static_cast<unsigned>(a.cout_pad / 32 / nb)), dim3(256), 0, stream, a);
 }
 
 KernelFn pick_halo8_stream_k() { return conv_halo8_sk_kernel; }

@@ -20,6 +20,7 @@ struct LeftTiles {
     const char *records;
     uint32_t *state;
     int32_t record, per;
+    int32_t whole;  // row tiles before those that are left in any case (all of them without such)
 };
 
 struct ConvArgs {
@@ -150,17 +151,19 @@ void launch_fold_plan(const int32_t *kmap, int64_t n_parents, void *plan, const 
 void launch_conv_fold(const ConvArgs &a, int nbw, hipStream_t stream);
 // The general kernels over the tiles of `rows` rows that the records (of `record`
 // bytes) leave over: the 64-row halo kernel of nb column blocks, and split-K
-// kernels (BF16: tiling 19 on 32-channel chunks; FP32: tiling 18, 13, 12 or 14 for
+// kernels (BF16: tiling 19 on 32-channel chunks, of whose tiles those from `tiles`
+// on are all left; FP32: tiling 18, 13, 12 or 14 for
 // nb 4, 3, 2 or 1).
 void launch_halo_left(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state, hipStream_t stream);
-void launch_splitk_left_bf16(ConvArgs a, int rows, const void *records, int record, uint32_t *state, hipStream_t stream);
+void launch_splitk_left_bf16(ConvArgs a, int rows, int64_t tiles, const void *records, int record, uint32_t *state,
+                             hipStream_t stream);
 void launch_splitk_left_f32(ConvArgs a, int nb, int rows, const void *records, int record, uint32_t *state,
                             hipStream_t stream);
 // BF16 convs over many rows, 96 columns a workgroup (conv_rows.hip): a record
-// per 512 rows.
 constexpr int kRowsRecord = 34816;
-void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, hipStream_t stream);
-void launch_conv_rows(const ConvArgs &a, hipStream_t stream);
+// per 512 rows; the first `tiles` of them, the others left to the general kernel.
+void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, int64_t tiles, void *plan, hipStream_t stream);
+void launch_conv_rows(const ConvArgs &a, int64_t tiles, hipStream_t stream);
 // The FP32 1x1-layer kernel reading BF16 rows, else nullptr.
 KernelFn pick_linear_f32_bf16_rows(int nbt);
 // The same on BF16 MFMAs with three-term split weights (Cin = 16 * ksx,
@@ -185,7 +188,13 @@ struct Frag<float> {
     static constexpr int E = 4;
 };
 
-// Whether a general kernel's row tile was left to it.
+// A workgroup's row tile in such a launch: XCD-contiguous runs (xcd_tile) of the tiles
+// that may be left and of those that are.
+__device__ __forceinline__ int left_tile(const LeftTiles &l) {
+    const int b = blockIdx.x;
+    return b < l.whole ? xcd_tile(b, l.whole) : l.whole + xcd_tile(b - l.whole, gridDim.x - l.whole);
+}
+// Whether it was left.
 __device__ __forceinline__ bool is_left(const LeftTiles &l, int tile) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) l.state[kFoldBadRows] = 0u;
     const uint32_t mode = *reinterpret_cast<const uint32_t *>(l.records + static_cast<int64_t>(tile / l.per) * l.record);
@@ -1485,7 +1494,7 @@ __device__ __forceinline__ void splitk_body(const ConvArgs &a) {
     if constexpr (MODE == kWholeTiles) {
         piece(xcd_tile(blockIdx.x, gridDim.x), blockIdx.y * NB, 0, INT32_MAX, nullptr);
     } else if constexpr (MODE == kLeftTiles) {
-        const int tile = xcd_tile(blockIdx.x, gridDim.x);
+        const int tile = left_tile(a.left);
         if (is_left(a.left, tile)) piece(tile, blockIdx.y * NB, 0, INT32_MAX, nullptr);
     } else {
         const int64_t tiles = (a.n_out + BM - 1) / BM;
@@ -1521,11 +1530,12 @@ __global__ void __launch_bounds__(256, MB == 4 ? 1 : 2) conv_splitk_left_kernel(
     splitk_body<T, NB, KC, 0, SUB, MB, kLeftTiles>(a);
 }
 template <class T, int NB, int KC, int SUB, int MB>
-void launch_left(ConvArgs &a, int rows, const void *records, int record, uint32_t *state, hipStream_t stream) {
-    a.left = LeftTiles{static_cast<const char *>(records), state, record, rows / (32 * MB)};
+void launch_left(ConvArgs &a, int rows, int64_t tiles, const void *records, int record, uint32_t *state, hipStream_t stream) {
+    const int per = rows / (32 * MB);
+    const int64_t row_tiles = (a.n_out + 32 * MB - 1) / (32 * MB);
+    a.left = LeftTiles{static_cast<const char *>(records), state, record, per, static_cast<int32_t>(std::min(row_tiles, tiles * per))};
     hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_splitk_left_kernel<T, NB, KC, SUB, MB>),
-                       dim3(static_cast<unsigned>((a.n_out + 32 * MB - 1) / (32 * MB)), static_cast<unsigned>(a.cout_pad / 32 / NB)),
-                       dim3(256), 0, stream, a);
+                       dim3(static_cast<unsigned>(row_tiles), static_cast<unsigned>(a.cout_pad / 32 / NB)), dim3(256), 0, stream, a);
 }
 
 // The tiles that a split-K kernel's stream-K runs left in parts: the pieces'

@@ -44,8 +44,8 @@ static_assert(kRowsRecord % 1024 == 0, "whole KiB");
 // Table entries: the offset of piece 0 in 16-byte units.
 __device__ __forceinline__ uint32_t rows_entry(uint32_t s) { return s * 4 + ((s >> 1) & 3); }
 
-// One workgroup per tile.
-__global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, int64_t n_out, int64_t n_src, char *plan) {
+// One workgroup per tile; tiles from `most` on are left to the general kernel.
+__global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, int64_t n_out, int64_t n_src, int most, char *plan) {
     constexpr int NTH = 1024, WORDS = 4096;  // a bitmap over 131,072 rows
     constexpr int V4 = kRowsTile * kMaxKvol / 4, Q = (V4 + NTH - 1) / NTH;
     __shared__ __align__(16) uint16_t table[kRowsTile * kMaxKvol];
@@ -55,6 +55,10 @@ __global__ void __launch_bounds__(1024) rows_plan_kernel(const int32_t *kmap, in
     __shared__ uint32_t sums[NTH / 64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    if (tile >= most) {
+        if (tid == 0) *reinterpret_cast<uint4 *>(plan + static_cast<int64_t>(tile) * kRowsRecord) = make_uint4(kFoldGeneral, 0u, 0u, 0u);
+        return;
+    }
     const int64_t m0 = static_cast<int64_t>(tile) * kRowsTile;
     const int count = static_cast<int>(min(static_cast<int64_t>(kRowsTile), n_out - m0)) * kMaxKvol;
     // 16-byte buffer loads that end at the map's last entry (zeros past it)
@@ -343,16 +347,14 @@ __global__ void __launch_bounds__(256, 1) conv_rows_kernel(ConvArgs a) {
 
 }  // namespace
 
-void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, void *plan, hipStream_t stream) {
+void launch_rows_plan(const int32_t *kmap, int64_t n_out, int64_t n_src, int64_t tiles, void *plan, hipStream_t stream) {
     hipLaunchKernelGGL(rows_plan_kernel, dim3(static_cast<unsigned>((n_out + kRowsTile - 1) / kRowsTile)), dim3(1024), 0,
-                       stream, kmap, n_out, n_src, static_cast<char *>(plan));
+                       stream, kmap, n_out, n_src, static_cast<int>(tiles), static_cast<char *>(plan));
 }
 
-void launch_conv_rows(const ConvArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL(conv_rows_kernel,
-                       dim3(static_cast<unsigned>((a.n_out + kRowsTile - 1) / kRowsTile),
-                            static_cast<unsigned>(a.cout_pad / 96)),
-                       dim3(256), 0, stream, a);
+void launch_conv_rows(const ConvArgs &a, int64_t tiles, hipStream_t stream) {
+    hipLaunchKernelGGL(conv_rows_kernel, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(a.cout_pad / 96)), dim3(256), 0,
+                       stream, a);
 }
 
 }  // namespace s3dx

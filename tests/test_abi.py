@@ -180,6 +180,12 @@ def test_conv_plan_names_the_mesh_layers_kernels(s3dx, monkeypatch):
     assert text(768, 192, s3dx.BF16, 300, 2400, True).startswith("pre=rows parent-rows mfma tiling=21 ")
     assert text(96, 96, s3dx.BF16, 64 * p, 64 * p, False) == \
         "pre=rows rows=512 cols=96 grid=3534x1 else mfma tiling=19 split-k rows=64 cols=96 kc=32 xf=0 ln=none grid=28265x1"
+    # whole passes over the CUs: the split-K kernel takes fewer than 96 tiles more
+    for tiles, taken in ((256, 256), (257, 256), (351, 256), (352, 352), (512, 512), (600, 512)):
+        n = 512 * tiles
+        assert f" rows=512 cols=96 grid={taken}x1 " in text(96, 96, s3dx.BF16, n, n, False), tiles
+    assert " rows=512 cols=96 grid=256x2 " in text(160, 192, s3dx.BF16, 512 * 257, 512 * 257, False)
+    assert " rows=512 " not in text(96, 96, s3dx.BF16, 512 * 255, 512 * 255, False)
     assert text(768, 192, s3dx.F32, 6001, 8 * 6001, True).startswith("pre=rows parent-rows fold terms=3 rows=512 cols=32 grid=94x6 else ")
     assert text(192, 192, s3dx.F32, 48008, 48008, False) == \
         "pre=rows mfma tiling=25 terms=3 rows=128 cols=64 kc=32 xf=0 ln=none grid=376x3 plan=own"
