@@ -248,7 +248,8 @@ S3DX_API s3dx_status s3dx_downsample_coords(const int32_t *coords, int64_t n, in
  * Arithmetic: float32 inputs use FP32 MFMA/VALU, or, in 3x3x3 layers with
  * records of the map at hand (a gather plan made for an FP32 layer, or input
  * transforms, whose layers make their own), BF16 MFMA on three BF16 terms of
- * every value, with no larger error against float64; bfloat16 inputs use BF16
+ * every value (at 2^24 times it; sums of 2^80 and more and rows of 2^104 and more
+ * take FP32 MFMA), with no larger error against float64; bfloat16 inputs use BF16
  * MFMA (layers that gather parent rows behind an input affine may multiply sums
  * of the weights that reach one parent, to 2^-27 of each sum); all accumulate in
  * float32.  Deterministic (no atomics on outputs).

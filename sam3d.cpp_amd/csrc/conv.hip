@@ -144,8 +144,9 @@ __global__ void __launch_bounds__(256) xform_rows_kernel(XformArgs a) {
             o = make_uint4(__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1]),
                            __builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3]));
             if (a.fold_state) {
-                // infinities, NaN, and what rounds to an infinite first term
-                auto none = [](uint32_t u) { return (u & 0x7fffffffu) >= 0x7f7f8000u; };
+                // infinities, NaN, and what rounds to an infinite first term (at 2^24
+                // times the value, conv_f3.hip)
+                auto none = [](uint32_t u) { return (u & 0x7fffffffu) >= 0x7f7f8000u - (24u << 23); };
                 if (none(o.x) || none(o.y) || none(o.z) || none(o.w)) a.fold_state[kFoldBadRows] = 1u;
             }
         }

@@ -51,8 +51,16 @@ constexpr int kF3Lds = kF3Flag + 16;
 static_assert(128 * 128 * 4 <= kF3Rec, "the output tile overlays the planes");
 static_assert(kF3Lds <= 160 * 1024, "LDS");
 
-// Three terms of two floats, packed (first value in the low half).
+// Rows and weights are split at 2^24 times their value and sums brought back: every
+// FP32 value, subnormal ones too, then has three normal terms (unscaled, values
+// below 2^-110 would lose low bits).  Values from 2^104 on, and sums from 2^80 on,
+// overflow at that scale: their tiles are done again with FP32 matrix instructions.
+constexpr float kF3Scale = 0x1p24f, kF3Unscale = 0x1p-48f;
+
+// Three terms of two (scaled) floats, packed (first value in the low half).
 __device__ __forceinline__ void split3(float a, float b, uint32_t (&t)[3]) {
+    a *= kF3Scale;
+    b *= kF3Scale;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         t[i] = pack_bf16x2(a, b);
@@ -443,17 +451,24 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
                 }
             }
         }
-        if (none) *flag = 1u;
-        __syncthreads();
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) hi[mb][r] += lo[mb][r];
+            for (int r = 0; r < 16; ++r) {
+                const float v = hi[mb][r] + lo[mb][r];
+                none = none || !(__builtin_fabsf(v) < __builtin_inff());
+                hi[mb][r] = v * kF3Unscale;
+            }
+        if (none) *flag = 1u;
+        __syncthreads();
     }
     if constexpr (FOLD) {
         // 32 columns of the slot's row of each parent, through this wave's 8 KiB
         // of LDS: 16-byte stores of 4 columns
-        __syncthreads();  // the planes are free
+        // (a sum that overflowed: the whole tile is left to the FP32 kernel behind)
+        if (*flag != 0u && tid == 0)
+            *const_cast<uint32_t *>(reinterpret_cast<const uint32_t *>(static_cast<const char *>(a.plan) +
+                                                                       static_cast<int64_t>(tile) * kGatherPlanRecord128)) = kFoldGeneral;
         float *stg = reinterpret_cast<float *>(smem) + wave * 64 * 33;
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
@@ -483,29 +498,41 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
     }
     if (__builtin_amdgcn_readfirstlane(*flag) != 0u) {
         // FP32 matrix instructions, rows from memory (k-steps of 8 channels,
-        // every KS-th one this wave's)
+        // every KS-th one this wave's); every fourth offset in a sum of its own, so
+        // that the sums are no longer than the FP32 kernels'
+        f32x16 sum[4][2];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) hi[mb] = f32x16{};
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) sum[j][mb] = f32x16{};
         const uint4 *w = static_cast<const uint4 *>(a.w);
-        for (uint32_t rest = mask; rest != 0u; rest &= rest - 1u) {
-            const int o = __builtin_ctz(rest);
-            int32_t row[2];
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-                const uint32_t v = table[o * ROWS + rg * 64 + mb * 32 + (lane & 31)];
-                const int sl = static_cast<int>(v >> 7);
-                row[mb] = mode != 0u ? static_cast<int32_t>(v)
-                                     : sl < distinct ? static_cast<int32_t>(slot_row[min(sl, kH8Single - 1)]) : -1;
-            }
-            for (int s = kp; s < a.cin / 8; s += KS) {
-                const uint4 b = w[(static_cast<int64_t>(o * (a.cin / 8) + s) * nbtot + nb0 + cb) * 64 + lane];
+        for (uint32_t rest = mask; rest != 0u;)
+            static_for<0, 4>([&](auto jc) __attribute__((always_inline)) {
+                constexpr int j = decltype(jc)::value;
+                if (rest == 0u) return;
+                const int o = __builtin_ctz(rest);
+                rest &= rest - 1u;
+                int32_t row[2];
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
-                    const uint4 v = gather_plain<float>(a.x, static_cast<int32_t>(a.x_bytes), row[mb], a.cin, s * 8 + half * 4);
-                    hi[mb] = mfma_step<float>(v, b, hi[mb]);
+                    const uint32_t v = table[o * ROWS + rg * 64 + mb * 32 + (lane & 31)];
+                    const int sl = static_cast<int>(v >> 7);
+                    row[mb] = mode != 0u ? static_cast<int32_t>(v)
+                                         : sl < distinct ? static_cast<int32_t>(slot_row[min(sl, kH8Single - 1)]) : -1;
                 }
-            }
-        }
+                for (int s = kp; s < a.cin / 8; s += KS) {
+                    const uint4 b = w[(static_cast<int64_t>(o * (a.cin / 8) + s) * nbtot + nb0 + cb) * 64 + lane];
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb) {
+                        const uint4 v = gather_plain<float>(a.x, static_cast<int32_t>(a.x_bytes), row[mb], a.cin, s * 8 + half * 4);
+                        sum[j][mb] = mfma_step<float>(v, b, sum[j][mb]);
+                    }
+                }
+            });
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) hi[mb][r] = (sum[0][mb][r] + sum[1][mb][r]) + (sum[2][mb][r] + sum[3][mb][r]);
     }
     __syncthreads();  // the planes become the output tile
 
@@ -568,7 +595,7 @@ __global__ void __launch_bounds__(256) f3_fold_weights_kernel(const float *w, ui
         bool none = false;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            double u = sum[2 * e], v = sum[2 * e + 1];
+            double u = kF3Scale * sum[2 * e], v = kF3Scale * sum[2 * e + 1];
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 t[e][j] = pack_bf16x2(static_cast<float>(u), static_cast<float>(v));

@@ -296,3 +296,44 @@ def test_plan_of_a_map_too_long_for_128_row_records(s3dx, W):
     gp = conv.gather_plan(n, kd, n)
     assert "terms=3" not in conv.plan(n, n, gp)
     s3dx.synchronize()
+
+
+@pytest.mark.parametrize("xs,ws", [(2.0 ** -120, 1.0), (1.0, 2.0 ** -120), (2.0 ** -130, 1.0), (2.0 ** -60, 2.0 ** -60), (2.0 ** 60, 2.0 ** 40)])
+def test_small_and_large_values(s3dx, O, W, xs, ws):
+    # Values whose third term is subnormal or below (or, at 2^-130, which are
+    # subnormal themselves), and sums that overflow at the kernel's scale: no larger
+    # an error than the FP32 instructions'.
+    coords = W.shells_union(0)[:9000]
+    n = coords.shape[0]
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, _ = _layer(s3dx, W, 64, 128, False)
+    w = (w * np.float32(ws)).astype(np.float32)
+    conv.set_weights(w, s3dx.WEIGHT_SLAT, None)
+    x = (W.normal_f32(91, 1, (n, 64)) * np.float32(xs)).astype(np.float32)
+    kd, xd = s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray.from_host(x)
+    gp = conv.gather_plan(n, kd, n)
+    assert "terms=3" in conv.plan(n, n, gp)
+    ys = [s3dx.DeviceArray((n, 128), np.float32) for _ in range(2)]
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32, plan=gp)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32)
+    ref = _ref(x, kmap, w, np.zeros(128))
+    e, f = (float(np.linalg.norm(y.download() - ref) / np.linalg.norm(ref)) for y in ys)
+    print(f"x {xs:.0e} w {ws:.0e}: rel-L2 three terms {e:.2e}, FP32 {f:.2e}", flush=True)
+    assert e <= 1.05 * f, (e, f)
+
+
+@pytest.mark.parametrize("ws", [2.0 ** -120, 2.0 ** 100])
+def test_folded_fp32_small_and_large_sums(s3dx, W, monkeypatch, ws):
+    p, cin, cout = 3001, 64, 96
+    conv, kmap, x, h, w, b = _mesh(s3dx, W, p, cin, cout, True)
+    w = (w * np.float32(ws)).astype(np.float32)
+    conv.set_weights(w, s3dx.WEIGHT_MESH, None)
+    assert " fold terms=3 " in conv.plan(p, 8 * p)
+    got = _run(s3dx, conv, x, kmap, cout)
+    monkeypatch.setenv("S3DX_CONV_TILING", "11")
+    fp32 = _run(s3dx, conv, x, kmap, cout)
+    monkeypatch.delenv("S3DX_CONV_TILING")
+    ref = _ref(h, np.where(kmap >= 0, kmap >> 3, -1), w, np.zeros(cout), mesh=True)
+    e, f = (float(np.linalg.norm(y - ref) / np.linalg.norm(ref)) for y in (got, fp32))
+    print(f"w {ws:.0e}: rel-L2 {e:.2e}, FP32 {f:.2e}", flush=True)
+    assert e <= 1.05 * f, (e, f)
