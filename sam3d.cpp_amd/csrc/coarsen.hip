@@ -154,12 +154,15 @@ window_assign_kernel(const int4 *__restrict__ coords, int32_t n, const uint32_t 
     __shared__ uint32_t wave_sums[kScanThreads / 64];
     __shared__ uint32_t prefix[kCoarseWords];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // (final: the marking is done; read beside the words, whose latency it shares)
+    const bool outside = flags[kOutside] != 0u;
     uint32_t counts[WPT], mine = 0;
 #pragma unroll
     for (int k = 0; k < WPT; ++k) {
         counts[k] = static_cast<uint32_t>(__popc(bitmap[tid * WPT + k]));
         mine += counts[k];
     }
+    if (outside) return;
     uint32_t incl = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -183,7 +186,7 @@ window_assign_kernel(const int4 *__restrict__ coords, int32_t n, const uint32_t 
     if (blockIdx.x == 0 && tid == 0) *total = static_cast<int32_t>(all);
     __syncthreads();
     const int32_t i = blockIdx.x * kScanThreads + tid;
-    if (i >= n || flags[kOutside] != 0u) return;
+    if (i >= n) return;
     const int4 c = coords[i];
     const int32_t cell = coarse_cell(c);
     const uint32_t w = static_cast<uint32_t>(cell) >> 5, bit = static_cast<uint32_t>(cell) & 31u;
