@@ -767,8 +767,8 @@ bool f3_shape(const s3dx_conv *conv) {
 // workgroups (one per CU) takes 8 and, per 32-channel chunk, 5 per column block
 // and 1.7; the FP32 kernels about 95 TFLOP/s over all 27 offsets and 4.
 // Measured, three terms against FP32: 128 -> 128 on 2,000 rows 35 / 23 us,
-// 4,000 37 / 37, 8,000 45 / 72, 28,265 133 / 226; 64 -> 64 on 5,000 21 / 20,
-// 10,366 23 / 28; 1024 -> 1024 on 300 235 / 224, 5,086 1,441 / 2,004.
+// 4,000 37 / 37, 8,000 45 / 72, 28,265 124-135 / 201-226; 64 -> 64 on 5,000 21 / 20,
+// 10,366 23 / 28; 1024 -> 1024 on 300 235 / 224, 5,086 1,441-1,473 / 2,004.
 int f3_blocks(const s3dx_conv *conv, int64_t n_out) {
     const int blocks = conv->cout_pad / 32, chunks = conv->cin / 32;
     const int64_t tiles = (n_out + 127) / 128, cus = device_cus();
@@ -877,7 +877,7 @@ int64_t fold_bytes_of(const s3dx_conv *conv) {
     int64_t bytes = 0;
     if (conv->dtype == S3DX_F32)
         bytes = f3_shape(conv) && (conv->w3 || !conv->weights_set) ? f3_fold_weight_bytes(conv->cin, conv->cout_pad) : 0;
-    else if (conv->cin % 64 == 0)
+    else if (conv->cin % 64 == 0 && (conv->cout % 128 == 0 || conv->cout % 96 == 0))  // the halo kernels' columns
         bytes = fold_weight_bytes(conv->cin, conv->cout_pad / 32);
     return bytes < (int64_t(1) << 31) ? bytes : 0;
 }

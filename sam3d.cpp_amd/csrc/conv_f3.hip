@@ -17,8 +17,8 @@
 // straight from memory.
 //
 // What bounds it: the BF16 matrix rate (six products: 128 -> 128 on 28,265
-// rows is 150 GFLOP in 133 us, 1.13 PFLOP/s; 1024 -> 1024 on 5,086 1.73 TFLOP
-// in 1,441 us, 1.2; a large BF16 product reaches 1.26 here); the split of the
+// rows is 150 GFLOP in 124-135 us, 1.1-1.2 PFLOP/s; 1024 -> 1024 on 5,086 1.73 TFLOP
+// in 1,473 us, 1.2; a large BF16 product reaches 1.26 here); the split of the
 // rows, about 2.5K of 44K cycles a chunk, is what is left between.  The FP32
 // kernels took 204-226 and 1,986-2,004 us.  64 rows x 32 columns a wave: each
 // weight fragment feeds two row blocks and each row fragment six products, so

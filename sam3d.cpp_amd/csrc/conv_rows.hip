@@ -15,7 +15,7 @@
 //
 // What bounds it: one wave per SIMD hides nothing between a chunk's ends and a
 // tile's, so the matrix units are busy 53% of the time.  96 -> 96 on 1.81M rows:
-// 880-940 us and the plan 110, against 1,372-1,434 for 64-row split-K tiles.
+// 845-950 us and the plan 100, against 1,372-1,434 for 64-row split-K tiles.
 // (Persistent workgroups that read the next tile's record and rows ahead took
 // 825-912; more weights in flight and other orders of the row reads, the same.
 // 192 -> 192 on 226,120 rows: 488 with the plan against 497 for the 64-row halo
