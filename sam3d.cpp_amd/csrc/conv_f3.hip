@@ -41,6 +41,7 @@ constexpr int kF3Chunk = 32;                               // channels per chunk
 constexpr int kF3MostRows = 719;                           // distinct rows that it stages at once
 constexpr int kF3Part = 712;                               // of more, the first (whole swizzle periods, one row fewer)
 constexpr int kF3Rows = kF3MostRows + 1;                   // rows a plane holds (the last is the zero row)
+constexpr int kF3Sum = 8;                                  // chunks of a sum
 constexpr int kF3Offsets = 5;                              // offsets of 128 rows that it stages at once
 static_assert(kF3Part % 8 == 0 && kF3Part < kF3MostRows && kH8Single - kF3Part < kF3Part, "two parts");
 static_assert(kF3Offsets * 128 <= kF3MostRows, "five offsets' rows");
@@ -156,9 +157,11 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
 
     const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.x), static_cast<short>(0),
                                                           static_cast<int32_t>(a.x_bytes), 0x00020000);
-    f32x16 hi[2], lo[2];
+    // (sums of kF3Sum chunks, which are then added to the total: 2048 channels
+    // added one after another had 1.03 times the FP32 kernels' error)
+    f32x16 hi[2], lo[2], total[2];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb) hi[mb] = lo[mb] = f32x16{};
+    for (int mb = 0; mb < 2; ++mb) hi[mb] = lo[mb] = total[mb] = f32x16{};
 
     bool none = false;  // a value without three finite terms was met
     if (mask != 0u) {
@@ -386,6 +389,13 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
                     }
                     if (i < n) products(aq[0], bq[0]);
                 }
+                if (cn != c && cn % kF3Sum == 0 && cn < chunks)
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) total[mb][r] += hi[mb][r];
+                        hi[mb] = f32x16{};
+                    }
                 c = cn;
                 q = qn;
             }
@@ -455,7 +465,7 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float v = hi[mb][r] + lo[mb][r];
+                const float v = (total[mb][r] + hi[mb][r]) + lo[mb][r];
                 none = none || !(__builtin_fabsf(v) < __builtin_inff());
                 hi[mb][r] = v * kF3Unscale;
             }

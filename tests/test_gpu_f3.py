@@ -337,3 +337,25 @@ def test_folded_fp32_small_and_large_sums(s3dx, W, monkeypatch, ws):
     e, f = (float(np.linalg.norm(y - ref) / np.linalg.norm(ref)) for y in (got, fp32))
     print(f"w {ws:.0e}: rel-L2 {e:.2e}, FP32 {f:.2e}", flush=True)
     assert e <= 1.05 * f, (e, f)
+
+
+def test_long_sums(s3dx, O, W):
+    # 2048 channels, 55,296 products an output: float64 on sampled rows.
+    coords = W.shells_union(0)[:20000]
+    n, cin, cout = coords.shape[0], 2048, 128
+    kmap = O.kmap_subm3(coords, n)
+    conv, w, b = _layer(s3dx, W, cin, cout, True)
+    x = np.random.default_rng(160).standard_normal((n, cin), np.float32)
+    kd, xd = s3dx.DeviceArray.from_host(kmap), s3dx.DeviceArray.from_host(x)
+    gp = conv.gather_plan(n, kd, n)
+    assert "terms=3 rows=128 cols=128" in conv.plan(n, n, gp)
+    ys = [s3dx.DeviceArray((n, cout), np.float32) for _ in range(2)]
+    conv.run(xd, n, kd, n, ys[0], s3dx.F32, plan=gp)
+    conv.run(xd, n, kd, n, ys[1], s3dx.F32)
+    rows = np.sort(np.random.default_rng(161).choice(n, 600, replace=False))
+    ref = _ref(x, kmap[rows], w, b)
+    ref = (ref - ref.mean(1, keepdims=True)) / np.sqrt(ref.var(1, keepdims=True) + 1e-6)
+    ref = ref / (1.0 + np.exp(-ref))
+    e, f = (rel_l2(y.download()[rows], ref) for y in ys)
+    print(f"2048 -> 128: rel-L2 three terms {e:.3e}, FP32 {f:.3e}", flush=True)
+    assert e <= f, (e, f)
