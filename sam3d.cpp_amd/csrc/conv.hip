@@ -886,9 +886,8 @@ int64_t fold_bytes_of(const s3dx_conv *conv) {
 // general kernel: a layer that reads repeated parent rows through an affine +
 // SiLU pass (so it has buffers of its own, see s3dx_conv_run) and writes rows
 // of its own type of all 8 children of every parent, with no LayerNorm or
-// residual.  BF16: where it would run the 64-row halo kernel (the BF16 output's
-// rounding hides the folding's); FP32: as three BF16 terms, 1.  What the map
-// holds is checked on the device.
+// residual.  BF16: where it would run the 64-row halo kernel; FP32: as three BF16
+// terms, 1.  What the map holds is checked on the device.
 int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_in, int64_t n_out,
                    bool residual, int32_t y_dtype) {
     if (!p.mfma || p.linear || !p.tl || p.xf || conv->kvol != kMaxKvol || src.shift != 3 || !conv->pre_scale ||

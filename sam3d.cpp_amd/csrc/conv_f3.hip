@@ -29,9 +29,9 @@
 // shells names about 470 in 128 rows, 534 at most, a solid bar of 24 x 24 x 60 up
 // to 768) are multiplied in two parts.  Tiles without slots (rows in no order) stage
 // five offsets' rows at a time, or, with fewer than 128 columns a workgroup, gather
-// rows from memory and split them in registers.  Tiles whose rows hold a value with no finite first
-// term (infinities, NaN) are done again with FP32 matrix instructions, so that
-// such values spread as in any FP32 sum.
+// rows from memory and split them in registers.  Tiles whose rows hold a value with
+// no finite first term (infinities, NaN), or whose sums overflow, are done again
+// with FP32 matrix instructions, so that such values spread as in any FP32 sum.
 #include "halo_tile.hpp"
 
 namespace s3dx {

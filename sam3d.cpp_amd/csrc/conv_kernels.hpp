@@ -133,7 +133,7 @@ int64_t f3_weight_bytes(int cin, int cout_pad);
 void launch_f3_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
 KernelFn pick_f3(int cg);
 // The same for folded parent rows: the folded weights' terms, and the folded
-// run with the FP32 pass over the listed tiles behind it.
+// kernel over a fold plan's records.
 int64_t f3_fold_weight_bytes(int cin, int cout_pad);
 void launch_f3_fold_weights(const void *w, void *out, int cin, int cout_pad, uint32_t *bad, hipStream_t stream);
 void launch_conv_f3_fold(const ConvArgs &a, hipStream_t stream);

@@ -105,7 +105,7 @@ def test_maps_no_subdivide_made(s3dx, W, monkeypatch):
 
 def test_infinities_new_weights_and_sizes(s3dx, W, monkeypatch):
     # An infinite or NaN row sends the run to the 27-offset kernel (the folded
-    # sum's two terms may differ in sign); the next run folds again.  New
+    # sum's terms may differ in sign); the next run folds again.  New
     # weights are folded anew; a larger set, then the first again.
     cin, cout = 192, 96
     conv, kmap, x, w, b, *_ = _setup(s3dx, W, W.shells_union(2)[:7000], cin, cout)
