@@ -891,7 +891,9 @@ int64_t fold_bytes_of(const s3dx_conv *conv) {
 int fold_blocks_of(const s3dx_conv *conv, const LaunchPlan &p, const Source &src, int64_t n_in, int64_t n_out,
                    bool residual, int32_t y_dtype) {
     if (!p.mfma || p.linear || !p.tl || p.xf || conv->kvol != kMaxKvol || src.shift != 3 || !conv->pre_scale ||
-        conv->ln || residual || y_dtype != conv->dtype || n_out != 8 * n_in || !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING") || n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
+        conv->ln || residual || y_dtype != conv->dtype || n_out != 8 * n_in ||
+        !aligned(conv->bias, 16) || std::getenv("S3DX_CONV_TILING") ||
+        n_out * kMaxKvol * 4 >= (int64_t(1) << 31) ||
         (n_in + 127) / 128 * kGatherPlanRecord128 >= (int64_t(1) << 31))
         return 0;
     if (!fold_bytes_of(conv) || (!conv->w_fold && conv->weights_set)) return 0;
