@@ -461,15 +461,21 @@ __global__ void __launch_bounds__(kHalo8Threads, 1) conv_f3_kernel(ConvArgs a) {
                 }
             }
         }
+        if (chunks > kF3Sum)
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) hi[mb][r] += total[mb][r];
+        float zero = 0.0f;  // (NaN once a sum is no finite number)
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float v = (total[mb][r] + hi[mb][r]) + lo[mb][r];
-                none = none || !(__builtin_fabsf(v) < __builtin_inff());
+                const float v = hi[mb][r] + lo[mb][r];
+                zero = __builtin_fmaf(v, 0.0f, zero);
                 hi[mb][r] = v * kF3Unscale;
             }
-        if (none) *flag = 1u;
+        if (none || zero != 0.0f) *flag = 1u;
         __syncthreads();
     }
     if constexpr (FOLD) {
